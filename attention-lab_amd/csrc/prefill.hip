@@ -396,9 +396,14 @@ __global__ __launch_bounds__(256) void project_keys_mfma(ProjectArgs a) {
 //                  column is its own query row, so the softmax state of a row lives in lanes n and n + 32
 //   P^T           online softmax in the log2 domain on the accumulators; the C layout of S^T is already the B
 //                  layout P^T needs for the next product (keys 8 (i/4) + 4 (l/32) + i%4 of row l%32)
-//   O^T += V^T P^T A = 32 dims x 16 keys from V^T in LDS (staged transposed, two keys per 32-bit word), B = P^T
-// O^T keeps each row's 128 outputs in the lanes of that row, so rescaling needs no exchange. The next block's K/V
-// is loaded into registers while the current one is computed.
+//   O^T += V^T P^T A = 32 dims x 16 keys read from the row-major V tile by the transposing LDS read, B = P^T
+// O^T keeps each row's 128 outputs in the lanes of that row, so rescaling needs no exchange. K and V tiles are copied
+// into LDS without passing through registers, one block ahead (two pairs of tiles, one barrier per block).
+// What bounds it: power. At B=1, G=8, h=4, T=L=8192 it runs 524 us (1.04 PFLOP/s) at a clock of 2.04 GHz (2.4 GHz at
+// light load); forms that need fewer cycles (all operand reads issued ahead, the next block's S^T under this block's
+// softmax) or more (one workgroup of 8 waves, 2.27 GHz) end at the same time within 2 %, and one workgroup per CU at
+// 2.41 GHz takes 657 us. The form before this one (K and V through registers, V transposed by 4-byte LDS stores, two
+// barriers per block) took 642 us; the 1000-token chunk after 29011 (h=2) went from 309 to 264 us.
 // ---------------------------------------------------------------------------------------------------------------
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2v_t __attribute__((ext_vector_type(2)));
@@ -423,16 +428,6 @@ constexpr int kPrefillMaxSplits = 16;
 
 constexpr int kPaRows = 128;          // (query, head) rows per workgroup: 4 waves x 32
 constexpr int kPaKeys = 64;           // keys per block
-constexpr int kPaKPitch = 128 + 8;    // bf16 per K row in LDS (272 bytes: 16-byte aligned rows)
-constexpr int kPaVPitch = 64 + 4;     // bf16 per V^T row in LDS (136 bytes)
-
-// V^T in LDS: row d (a head dim) holds the block's 64 keys as 16 groups of 4 (8 bytes); group g of row d sits at slot
-// g ^ ((d >> 4) & 7). The staging store of a wave writes 16 rows 8 apart, which without the permutation land on 4 of
-// the 32 banks (8-way conflicts); with it they cover all 32. The MFMA reads (32 consecutive rows, one group) keep one
-// permutation per 16 rows and stay conflict-free.
-__device__ __forceinline__ int vt_at(int d, int key) {
-    return d * kPaVPitch + ((((key >> 2) ^ (d >> 4)) & 15) << 2) + (key & 3);
-}
 constexpr float kPaLazy = 8.0f;       // rescale O only when the running max grows by more than 2^8
 
 // two fp32 -> packed bf16 pair, round to nearest even (gfx950 converts in hardware: v_cvt_pk_bf16_f32)
@@ -442,23 +437,56 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float x, float y) {
     return __builtin_bit_cast(uint32_t, v);
 }
 
-// two workgroups per CU: the register budget then fits without AGPRs (230 VGPRs), and one workgroup's softmax
-// hides the other's matrix-core latency (1.2-1.3x over one workgroup per CU)
+// 16 bytes per lane from global memory straight into LDS: the wave's 64 lanes fill the 1 KB at `lds` in lane order.
+__device__ __forceinline__ void load_lds16(const uint16_t* src, uint16_t* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// The same from a buffer of `bytes` bytes at `base` (wave-uniform), lane l from byte offset `off`; zeros past the end.
+__device__ __forceinline__ void load_lds16_buf(const uint16_t* base, uint32_t bytes, uint32_t off, uint16_t* lds) {
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, (int)bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)lds, 16, (int)off, 0, 0, 0);
+}
+
+// the larger of x over lanes l and l ^ 32 (v_permlane32_swap, no LDS round trip)
+__device__ __forceinline__ float max_xor32(float x) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Transposing LDS read (ds_read_b64_tr_b16): each 16 lanes read a 4 x 16 matrix of 16-bit elements, lane 4 e + j the
+// elements 4 j .. 4 j + 3 of row e; lane i receives column i.
+typedef short s16x4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x2v_t read_tr16(const char* lds) {
+    return __builtin_bit_cast(u32x2v_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                            (__attribute__((address_space(3))) s16x4_t*)lds));
+}
+
+// K and V blocks in LDS: 64 rows of 256 bytes, sixteen 16-byte chunks each, copied by load_lds16 (no registers, no
+// store instructions), so a row's chunks can only be permuted, not padded. K: chunk c of row j at slot c ^ (j & 15):
+// an MFMA operand read (16 rows, one chunk) covers all 64 banks. V: chunk c of row j at slot c ^ (4 (j & 3)): a
+// transposing read takes 32 dims (4 chunks) of 4 consecutive rows, which then lie in 4 different quarters of the banks.
+
+// two workgroups per CU: the register budget then fits without AGPRs, and one workgroup's softmax hides the other's
+// matrix-core latency (1.2-1.3x over one workgroup per CU)
 template <bool SPLIT>   // SPLIT: a.splits > 1, partials to a.part (the one-pass instance keeps no split logic)
 __global__ __launch_bounds__(256, 2) void prefill_attend(PrefillAttendArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t ks[kPaKeys * kPaKPitch];
-    __shared__ __attribute__((aligned(16))) uint16_t vt[128 * kPaVPitch];
+    __shared__ __attribute__((aligned(1024))) uint16_t kt0[kPaKeys * 128], vt0[kPaKeys * 128];
+    __shared__ __attribute__((aligned(1024))) uint16_t kt1[kPaKeys * 128], vt1[kPaKeys * 128];
     const int lin = xcd_contiguous_block();
     // the query tiles of a (b, g) in reverse: the later tiles read more keys, so they are dispatched first and the
     // short ones fill in behind them; the key splits of a tile are adjacent
     const int nsp = SPLIT ? a.splits : 1;
     const int per_bg = a.qtiles * nsp;
-    const int bg = lin / per_bg, rem = lin - bg * per_bg;
-    const int qt = a.qtiles - 1 - rem / nsp, sp = rem - (rem / nsp) * nsp;
+    const int bg = __builtin_amdgcn_readfirstlane(lin / per_bg), rem = lin - bg * per_bg;
+    const int rq = __builtin_amdgcn_readfirstlane(rem / nsp);
+    const int qt = a.qtiles - 1 - rq, sp = rem - rq * nsp;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31, g = lane >> 5;
-    const int BQ = kPaRows / a.h;
+    const int BQ = __builtin_amdgcn_readfirstlane(kPaRows / a.h);
     const int t0 = qt * BQ;
     const int R = 32 * wave + n;                 // this lane's row: query t0 + R / h, head R % h
     const int t = t0 + R / a.h, head = R % a.h;
@@ -474,47 +502,53 @@ __global__ __launch_bounds__(256, 2) void prefill_attend(PrefillAttendArgs a) {
     const int kend_tile = min(a.legal, a.q_pos0 + min(t0 + BQ, a.T));
     const int kb0 = SPLIT ? sp * a.kspan : 0;
     const int kend = SPLIT ? min(kend_tile, kb0 + a.kspan) : kend_tile;
-    const int wave_first = a.q_pos0 + min(t0 + (32 * wave) / a.h, a.T - 1);
-    const int kend_wave = min(a.legal, a.q_pos0 + min(t0 + (32 * wave + 31) / a.h, a.T - 1) + 1);
+    const int wave_first = a.q_pos0 + min(t0 + __builtin_amdgcn_readfirstlane((32 * wave) / a.h), a.T - 1);
+    const int kend_wave =
+        min(a.legal, a.q_pos0 + min(t0 + __builtin_amdgcn_readfirstlane((32 * wave + 31) / a.h), a.T - 1) + 1);
 
     const uint16_t* Kb = a.K + (size_t)bg * a.kv_bg_stride;
     const uint16_t* Vb = a.V + (size_t)bg * a.kv_bg_stride;
-    // staging: K chunk c = tid + 256 u -> key c / 16, 16 bytes at dim 8 (c % 16); V unit w = tid + 256 u -> dims
-    // 8 (w % 16) .. + 7 of keys 2 (w / 16) and 2 (w / 16) + 1 (16 lanes read one key's 256 bytes)
-    u32x4_t kr[4], vr[2][2];
-    auto gload = [&](int kb) {
+    // staging: load u of wave w fills rows 16 u + 4 w .. + 3 of a tile, lane l slot l % 16 of row 16 u + 4 w + l / 16. A
+    // load has a buffer of its own, the 4 rows it reads (rows past the range give zeros), so its address arithmetic is
+    // scalar; rows further apart than a 32-bit offset reaches take per-lane addresses (the last row past the range).
+    const int srow = 4 * wave + (lane >> 4);
+    const int kchunk = 8 * ((lane & 15) ^ srow), vchunk = 8 * ((lane & 15) ^ ((lane >> 4) << 2));
+    const uint32_t roff = (uint32_t)(lane >> 4) * (uint32_t)a.kv_row_stride;
+    const uint32_t koff = 2u * (roff + (uint32_t)kchunk), voff = 2u * (roff + (uint32_t)vchunk);
+    auto gload = [&](int kb, uint16_t* kt, uint16_t* vt) {
+        if (a.kv_row_stride < 1 << 28) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int c = tid + 256 * u;
-            const int key = min(kb + (c >> 4), kend - 1);
-            kr[u] = *reinterpret_cast<const u32x4_t*>(Kb + (size_t)key * a.kv_row_stride + 8 * (c & 15));
-        }
+            for (int u = 0; u < 4; ++u) {
+                const int row = kb + 16 * u + 4 * wave;
+                const size_t off = (size_t)row * a.kv_row_stride;
+                const int rows = __builtin_amdgcn_readfirstlane(max(min(kend - row, 4), 0));
+                const uint32_t bytes = 2u * (uint32_t)a.kv_row_stride * (uint32_t)rows;
+                load_lds16_buf(Kb + off, bytes, koff, kt + (16 * u + 4 * wave) * 128);
+                load_lds16_buf(Vb + off, bytes, voff, vt + (16 * u + 4 * wave) * 128);
+            }
+        } else {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int w = tid + 256 * u;
-            const int k0 = min(kb + 2 * (w >> 4), kend - 1), k1 = min(kb + 2 * (w >> 4) + 1, kend - 1);
-            vr[u][0] = *reinterpret_cast<const u32x4_t*>(Vb + (size_t)k0 * a.kv_row_stride + 8 * (w & 15));
-            vr[u][1] = *reinterpret_cast<const u32x4_t*>(Vb + (size_t)k1 * a.kv_row_stride + 8 * (w & 15));
-        }
-    };
-    auto lds_store = [&]() {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int c = tid + 256 * u;
-            *reinterpret_cast<u32x4_t*>(&ks[(c >> 4) * kPaKPitch + 8 * (c & 15)]) = kr[u];
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int w = tid + 256 * u;
-            const int kp = w >> 4, d0 = 8 * (w & 15);
-            const uint32_t x[4] = {vr[u][0].x, vr[u][0].y, vr[u][0].z, vr[u][0].w};
-            const uint32_t y[4] = {vr[u][1].x, vr[u][1].y, vr[u][1].z, vr[u][1].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {   // dims d0 + 2e, d0 + 2e + 1: (key 2kp, key 2kp + 1) pairs
-                *reinterpret_cast<uint32_t*>(&vt[vt_at(d0 + 2 * e, 2 * kp)]) = (x[e] & 0xffffu) | (y[e] << 16);
-                *reinterpret_cast<uint32_t*>(&vt[vt_at(d0 + 2 * e + 1, 2 * kp)]) = (x[e] >> 16) | (y[e] & 0xffff0000u);
+            for (int u = 0; u < 4; ++u) {
+                const size_t row = (size_t)min(kb + 16 * u + srow, kend - 1) * a.kv_row_stride;
+                load_lds16(Kb + row + kchunk, kt + (16 * u + 4 * wave) * 128);
+                load_lds16(Vb + row + vchunk, vt + (16 * u + 4 * wave) * 128);
             }
         }
+    };
+    // operand reads, as byte offsets into a tile: K row 32 kt + n, chunk 2 kk + g; V rows 16 ks + 8 hf + 4 g + e, dims
+    // 32 dt + 16 (lane / 16 % 2) + 4 j .. + 3, e = lane % 16 / 4, j = lane % 4. `pin` keeps the compiler from holding a
+    // copy of each per tile.
+    uint32_t kof[8], vof[4];
+    const int ve = (lane >> 2) & 3;
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) kof[kk] = 256 * n + 16 * ((2 * kk) ^ g ^ (n & 15));
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) vof[dt] = 256 * (4 * g + ve) + 64 * (dt ^ ve) + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+    auto pin = [&]() {
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) asm volatile("" : "+v"(kof[kk]));
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) asm volatile("" : "+v"(vof[dt]));
     };
 
     float m_run = -INFINITY, l_run = 0.0f;
@@ -533,44 +567,38 @@ __global__ __launch_bounds__(256, 2) void prefill_attend(PrefillAttendArgs a) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
 
-    if (kb0 < kend) gload(kb0);
-    for (int kb = kb0; kb < kend; kb += kPaKeys) {
-        if (kb != kb0) __syncthreads();   // the previous block's LDS reads are done
-        lds_store();
-        __syncthreads();
-        if (kb + kPaKeys < kend) gload(kb + kPaKeys);
-        if (kb >= kend_wave) continue;   // every row of this wave ends before the block (no barrier skipped: the
-                                         // loop's barriers are at its top)
+    auto block = [&](int kb, const uint16_t* ks, const uint16_t* vs) {
         f32x16_t s[2];
 #pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
+        for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) s[kt][i] = 0.0f;
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                const bf16x8_t ka = __builtin_bit_cast(
-                    bf16x8_t, *reinterpret_cast<const u32x4_t*>(&ks[(32 * kt + n) * kPaKPitch + 16 * kk + 8 * g]));
+        for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const bf16x8_t ka = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t*>(
+                                                                     reinterpret_cast<const char*>(ks) + 8192 * kt + kof[kk]));
                 s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka, qb[kk], s[kt], 0, 0, 0);
             }
-        }
         // this lane's scores: row R, keys kb + 32 kt + 8 (i / 4) + 4 g + i % 4. The scale is positive here (a negative
         // one flipped the query's sign), so the block's largest scaled score comes from the raw scores and the scale
         // costs one multiply per row here and rides in the exponent's FMA below.
-        const bool full = kb + kPaKeys - 1 <= wave_first && kb + kPaKeys <= a.legal;   // no key of the block masked
+        if (!(kb + kPaKeys - 1 <= wave_first && kb + kPaKeys <= a.legal)) {   // a key of the block is masked
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = kb + 32 * kt + 8 * (i >> 2) + 4 * g + (i & 3);
+                    if (key > pos || key >= a.legal) s[kt][i] = -INFINITY;
+                }
+        }
         float bm = -INFINITY;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float v = s[kt][i];
-                if (!full) {
-                    const int key = kb + 32 * kt + 8 * (i >> 2) + 4 * g + (i & 3);
-                    if (key > pos || key >= a.legal) v = -INFINITY;
-                }
-                s[kt][i] = v;
-                bm = fmaxf(bm, v);
-            }
-        bm = fmaxf(bm, shfl_xor_f32(bm, 32)) * sc;
+            for (int i = 0; i < 16; ++i) bm = fmaxf(bm, s[kt][i]);
+        bm = max_xor32(bm) * sc;
         if (bm > m_run + kPaLazy) {   // also the first block of the row (m_run = -inf)
             const float al = fast_exp2(m_run - bm);   // exp2(-inf) = 0
             l_run *= al;
@@ -584,15 +612,22 @@ __global__ __launch_bounds__(256, 2) void prefill_attend(PrefillAttendArgs a) {
         // 8 (ks % 2) .. + 7, i.e. keys 16 (ks % 2) + 4 g + {0..3, 8..11} of the tile. p = exp2(scale * s - m): one
         // FMA and the exponential.
         bf16x8_t pb[4];
-        const float nm = -m_run;
+        const bool none = m_run == -INFINITY;   // no key of the row yet, or only NaN scores: every weight is zero
+        if (__any(none)) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s[kt][i] = none ? -INFINITY : s[kt][i];
+        }
+        const float nm = none ? 0.0f : -m_run;
 #pragma unroll
         for (int ks2 = 0; ks2 < 4; ++ks2) {
             uint32_t w4[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float x0 = s[ks2 >> 1][8 * (ks2 & 1) + 2 * e], x1 = s[ks2 >> 1][8 * (ks2 & 1) + 2 * e + 1];
-                const float p0 = m_run == -INFINITY ? 0.0f : fast_exp2(fmaf(x0, sc, nm));
-                const float p1 = m_run == -INFINITY ? 0.0f : fast_exp2(fmaf(x1, sc, nm));
+                const float p0 = fast_exp2(fmaf(x0, sc, nm));
+                const float p1 = fast_exp2(fmaf(x1, sc, nm));
                 l_run += p0 + p1;
                 w4[e] = pack_bf16x2(p0, p1);
             }
@@ -600,15 +635,32 @@ __global__ __launch_bounds__(256, 2) void prefill_attend(PrefillAttendArgs a) {
         }
 #pragma unroll
         for (int ks2 = 0; ks2 < 4; ++ks2) {
-            const int key0 = 32 * (ks2 >> 1) + 16 * (ks2 & 1) + 4 * g;
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
-                const u32x2v_t lo4 = *reinterpret_cast<const u32x2v_t*>(&vt[vt_at(32 * dt + n, key0)]);
-                const u32x2v_t hi4 = *reinterpret_cast<const u32x2v_t*>(&vt[vt_at(32 * dt + n, key0 + 8)]);
+                const char* vp = reinterpret_cast<const char*>(vs) + 4096 * ks2 + vof[dt];
+                const u32x2v_t lo4 = read_tr16(vp), hi4 = read_tr16(vp + 8 * 256);
                 const bf16x8_t va = __builtin_bit_cast(bf16x8_t, u32x4_t{lo4.x, lo4.y, hi4.x, hi4.y});
                 o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[ks2], o[dt], 0, 0, 0);
             }
         }
+    };
+    // Two tile pairs in LDS: a block's copies are issued as soon as every wave has left the tiles they overwrite (the
+    // barrier that also publishes the current block), and land while the current block is computed. The pairs are
+    // separate arrays, so that the compiler knows a block's reads apart from the copies in flight.
+    auto publish = [&]() {
+        __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this wave's copies have landed, its reads are done
+        asm volatile("s_barrier" ::: "memory");
+        pin();
+    };
+    if (kb0 < kend) gload(kb0, kt0, vt0);
+    for (int kb = kb0; kb < kend; kb += 2 * kPaKeys) {
+        publish();
+        if (kb + kPaKeys < kend) gload(kb + kPaKeys, kt1, vt1);
+        if (kb < kend_wave) block(kb, kt0, vt0);
+        if (kb + kPaKeys >= kend) break;
+        publish();
+        if (kb + 2 * kPaKeys < kend) gload(kb + 2 * kPaKeys, kt0, vt0);
+        if (kb + kPaKeys < kend_wave) block(kb + kPaKeys, kt1, vt1);
     }
     const float l_tot = l_run + shfl_xor_f32(l_run, 32);
     if (t >= a.T) return;

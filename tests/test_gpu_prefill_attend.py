@@ -175,3 +175,35 @@ def test_key_split_validation(gpu):
         nat.call("attnlab_prefill_attend_split", q.data_ptr(), K.data_ptr(), V.data_ptr(), 16 * 128, 128,
                  out.data_ptr(), 1, 1, 2, 4, 128, 0, 16, 16, 0.1, 2, part.data_ptr(), (need // 4 - 1) * 4,
                  nat.stream_of(gpu))
+
+
+@pytest.mark.parametrize("legal", [1, 31, 33, 63, 64, 65, 96, 127, 129, 192, 449])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_rows_past_the_range_are_never_read(gpu, legal, splits):
+    """K/V tiles are copied in whole 64-row blocks; rows at and past valid_length hold NaN here and must not reach any
+    output: bit for bit the read of the same cache with zeros there, at the edges of a block and of a 4-row copy."""
+    B, G, h, T, C = 2, 2, 2, min(legal, 70), legal + 70
+    K, V, q = inputs(gpu, B, G, h, T, C, seed=legal)
+    outs = []
+    for fill in (0.0, float("nan")):
+        K[:, :, legal:], V[:, :, legal:] = fill, fill
+        outs.append(hip_attend.prefill_attend(q, K, V, legal - T, legal, splits=splits))
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    check(outs[1], exact.causal_attention(f64(q), f64(K), f64(V), legal, list(range(legal - T, legal))), f"legal={legal}")
+
+
+def test_rows_further_apart_than_a_buffer_offset(gpu):
+    """A row stride past what the 4-row copies address with 32 bits (2^28 elements, half a GiB): the per-lane addresses
+    give the contiguous read's output bit for bit."""
+    h, T, legal, stride = 2, 3, 3, 1 << 28
+    K, V, q = inputs(gpu, 1, 1, h, T, legal, seed=7)
+    want = hip_attend.prefill_attend(q, K, V, 0, legal)
+    far = torch.empty(2 * stride + 256, dtype=torch.bfloat16, device=gpu)
+    for j in range(legal):
+        far[j * stride:j * stride + 128], far[j * stride + 128:j * stride + 256] = K[0, 0, j], V[0, 0, j]
+    out = torch.empty_like(want)
+    nat.call("attnlab_prefill_attend", q.data_ptr(), far.data_ptr(), far.data_ptr() + 256, 0, stride, out.data_ptr(), 1, 1,
+             h, T, 128, 0, legal, legal, 1.0 / math.sqrt(128), nat.stream_of(q.device))
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
