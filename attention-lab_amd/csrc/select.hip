@@ -294,28 +294,39 @@ __device__ __forceinline__ const uint64_t* radix_sort_desc_1024(SelectShared& sh
     return base + 1024 * cur;
 }
 
-// Score order for k <= 1024 staged pairs in slots [0, k) (one per thread), when the keys spread out: one pass into
-// 2048 bins that are linear in the key over [kmin, kmax] (bin = (kmax - key) >> s, with s the smallest shift that
-// leaves at most 2048 bins, so bin order is descending key order), then each pair's rank inside its bin by comparison
-// with the bin's other pairs, larger (key, ~index) first (equal pairs, which only zero padding can form, by their
-// place in the bin). Six barriers in all, against four per pass of the radix sort. The top k of a smooth score
-// distribution puts a few pairs in a bin; when a bin holds more than kBinSortMax (ties, outliers that stretch the key
-// range), nothing has been moved yet and the function returns nullptr for the caller's other sort. Counts in sh.hist;
-// bin starts and cursors in sortbuf[2048, 4096) (as uint32); pairs placed by bin in sortbuf[1024, 2048), sorted into
-// sortbuf[0, k).
+// Score order for k <= 1024 E staged pairs in slots [0, k), when the keys spread out: one pass into 4096 bins that are
+// linear in the key over [kmin, kmax] (bin = (kmax - key) >> s, with s the smallest shift that leaves at most 4096 bins,
+// so bin order is descending key order), then each pair's rank inside its bin by comparison with the bin's other pairs,
+// larger (key, ~index) first (pairs are distinct: their indices are; only slots that a histogram which does not match
+// the scores left at zero could be equal, and those may then repeat or miss a pair). The top k of a smooth score distribution puts a few
+// pairs in a bin; when a bin holds more than kBinSortMax (ties, outliers that stretch the key range), nothing has been
+// moved yet and the function returns false for the caller's other sort. The pairs wait in registers (E per thread)
+// between the phases, so they are sorted in place; the bins are 16-bit counters, two per word of sh.hist, turned into
+// each bin's first slot and then counted up to its end, which is the next bin's first slot.
+// What bounds it is a chain of LDS latencies (eight barriers), where the radix sort makes four passes of ballots and
+// scans and the bitonic sort of 8192 pairs 40 barriers. Tiled top-k in score order, eight rows of 128K scores: k = 4096
+// 52.4 -> 35.4 us, k = 8192 100.6 -> 46.0 (position order: 27.5, 34.0); eight rows of 64K, k = 2048: 35.4 -> 26.2.
 constexpr uint32_t kBinSortMax = 48;
-__device__ __forceinline__ const uint64_t* bin_sort_desc_1024(SelectShared& sh, int k) {
-    static_assert(kHistBins == 2 * kSelThreads, "two bins per thread");
+constexpr int kSortBins = 2 * kHistBins;
+template <int E>
+__device__ __forceinline__ bool bin_sort_desc(SelectShared& sh, int k) {
+    static_assert(kSortBins == 4 * kSelThreads, "two words of two bins per thread");
+    static_assert(E * kSelThreads <= 0xffff, "16-bit slots");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     uint64_t* const buf = sh.sortbuf;
     uint32_t* const cnt = sh.hist;
-    uint32_t* const start = reinterpret_cast<uint32_t*>(buf + 2048);
-    uint32_t* const cur = start + kHistBins;
-    uint64_t* const tmp = buf + 1024;
-    const bool valid = tid < k;
-    const uint64_t x = valid ? buf[tid] : 0ull;
-    const uint32_t key = (uint32_t)(x >> 32);
-    uint32_t mn = valid ? key : 0xffffffffu, mx = valid ? key : 0u;
+    const uint16_t* const end = reinterpret_cast<const uint16_t*>(sh.hist);
+    uint64_t x[E];
+    uint32_t mn = 0xffffffffu, mx = 0u;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int i = kSelThreads * e + tid;
+        x[e] = i < k ? buf[i] : 0ull;
+        if (i < k) {
+            mn = min(mn, (uint32_t)(x[e] >> 32));
+            mx = max(mx, (uint32_t)(x[e] >> 32));
+        }
+    }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) {
         mn = min(mn, (uint32_t)__shfl_xor((int)mn, m, 64));
@@ -335,15 +346,21 @@ __device__ __forceinline__ const uint64_t* bin_sort_desc_1024(SelectShared& sh, 
         kmax = max(kmax, sh.wave_tot[w][1]);
     }
     const uint32_t span = kmax - kmin;   // k >= 1, so kmin <= kmax
-    const int shift = span >> 11 ? 32 - __clz((int)span) - 11 : 0;
-    const uint32_t bin = (kmax - key) >> shift;   // < 2048
-    if (valid) atomicAdd(&cnt[bin], 1u);
+    const int shift = span >> 12 ? 32 - __clz((int)span) - 12 : 0;
+    auto bin_of = [&](uint64_t v) { return (kmax - (uint32_t)(v >> 32)) >> shift; };   // < 4096
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (kSelThreads * e + tid < k) {
+            const uint32_t b = bin_of(x[e]);
+            atomicAdd(&cnt[b >> 1], 1u << (16 * (b & 1u)));
+        }
     __syncthreads();
-    // exclusive scan of the 2048 counts (thread t: bins 2t, 2t + 1) and the largest count
+    // exclusive scan of the 4096 counts (thread t: bins 4t .. 4t + 3) and the largest count
     const uint2 c2 = reinterpret_cast<const uint2*>(cnt)[tid];
-    const uint32_t s2 = c2.x + c2.y;
-    const uint32_t inc = wave_incl_scan(s2);
-    uint32_t big = max(c2.x, c2.y);
+    const uint32_t c0 = c2.x & 0xffffu, c1 = c2.x >> 16, c2l = c2.y & 0xffffu, c3 = c2.y >> 16;
+    const uint32_t s4 = (c0 + c1) + (c2l + c3);
+    const uint32_t inc = wave_incl_scan(s4);
+    uint32_t big = max(max(c0, c1), max(c2l, c3));
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) big = max(big, (uint32_t)__shfl_xor((int)big, m, 64));
     __syncthreads();   // every thread has read the minimum and maximum out of wave_tot
@@ -358,29 +375,36 @@ __device__ __forceinline__ const uint64_t* bin_sort_desc_1024(SelectShared& sh, 
     }
     if (largest > kBinSortMax) {
         __syncthreads();   // the other sort reuses wave_tot
-        return nullptr;
+        return false;
     }
-    const uint32_t e0 = before + inc - s2;
-    reinterpret_cast<uint2*>(start)[tid] = make_uint2(e0, e0 + c2.x);
-    reinterpret_cast<uint2*>(cur)[tid] = make_uint2(e0, e0 + c2.x);
-    __syncthreads();
-    uint32_t pos = 0u;
-    if (valid) {
-        pos = atomicAdd(&cur[bin], 1u);
-        tmp[pos] = x;
-    }
-    __syncthreads();
-    if (valid) {
-        const uint32_t b0 = start[bin], b1 = cur[bin];
-        uint32_t rank = 0u;
-        for (uint32_t j = b0; j < b1; ++j) {
-            const uint64_t y = tmp[j];
-            rank += (y > x) || (y == x && j < pos);
+    const uint32_t e0 = before + inc - s4, e1 = e0 + c0, e2 = e1 + c1, e3 = e2 + c2l;
+    reinterpret_cast<uint2*>(cnt)[tid] = make_uint2(e0 | (e1 << 16), e2 | (e3 << 16));
+    __syncthreads();   // also: every pair is in registers
+    uint32_t pos[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        pos[e] = 0u;
+        if (kSelThreads * e + tid < k) {
+            const uint32_t b = bin_of(x[e]);
+            pos[e] = (atomicAdd(&cnt[b >> 1], 1u << (16 * (b & 1u))) >> (16 * (b & 1u))) & 0xffffu;
+            buf[pos[e]] = x[e];
         }
-        buf[b0 + rank] = x;
     }
     __syncthreads();
-    return buf;
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (kSelThreads * e + tid < k) {
+            const uint32_t b = bin_of(x[e]);
+            const uint32_t b0 = b ? end[b - 1] : 0u, b1 = end[b];
+            pos[e] = b0;
+            for (uint32_t j = b0; j < b1; ++j) pos[e] += buf[j] > x[e];
+        }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (kSelThreads * e + tid < k) buf[pos[e]] = x[e];
+    __syncthreads();
+    return true;
 }
 
 // Score order for 1024 < sort_len(k) <= 4096 staged pairs: the same stable LSD radix sort (passes of 8 bits, each
@@ -511,15 +535,16 @@ __device__ __forceinline__ void finish_row(const SelectArgs& a, int row, SelectS
     // descending on (key, ~index): larger score first, then lower index (sortbuf[0, sort_len(k)) was pre-filled by
     // init_sortbuf before the emission)
     __syncthreads();
-    // 128 pairs: the bitonic sort (one chunk pass in registers). 256 to 1024: the bin sort, or where its bins crowd
-    // the bitonic sort (256) or the radix sort (512, 1024). 1025 to 4096: the radix sort by sub-blocks; past 4096 the
-    // bitonic sort. Single-workgroup top-k on MI355X, score order's cost over position order per launch, 32K keys:
-    // k = 1024 3.7 us (radix sort alone 6.0), k = 512 3.3 (radix 4.3), k = 128 2.6 (bitonic; radix 4.0).
-    const uint64_t* sorted = nullptr;
+    // Up to 128 pairs: the bitonic sort (one chunk pass in registers). More: the bin sort, or where its bins crowd the
+    // bitonic sort (256, and past 4096), the radix sort (512, 1024) or the radix sort by sub-blocks (1025 to 4096).
+    // Single-workgroup top-k on MI355X, score order's cost over position order per launch, 32K keys: k = 1024 3.7 us
+    // (radix sort alone 6.0), k = 512 3.3 (radix 4.3), k = 128 2.6 (bitonic; radix 4.0).
+    const uint64_t* sorted = sh.sortbuf;
     const int n = sort_len(k);
-    if (n > 128 && n <= kSelThreads) sorted = bin_sort_desc_1024(sh, k);
-    if (sorted == nullptr) {
-        sorted = sh.sortbuf;
+    const bool binned = n <= 128 ? false
+                        : n <= kSelThreads ? bin_sort_desc<1>(sh, k)
+                        : n <= 4 * kSelThreads ? bin_sort_desc<4>(sh, k) : bin_sort_desc<8>(sh, k);
+    if (!binned) {
         if (n > 256 && n <= kSelThreads) sorted = radix_sort_desc_1024(sh, k);
         else if (n > kSelThreads && n <= 4 * kSelThreads) sorted = radix_sort_desc_4096(sh, k);
         else bitonic_sort_desc(sh.sortbuf, n);
@@ -821,7 +846,7 @@ __device__ __forceinline__ void for_each_chunk(const float* s, int M, int c_begi
     }
 }
 
-__device__ void select_row_streaming(const SelectArgs& a, int row, SelectShared& sh, const StreamLds& L) {
+__device__ __forceinline__ void select_row_streaming(const SelectArgs& a, int row, SelectShared& sh, const StreamLds& L) {
     const int tid = threadIdx.x;
     const int M = a.M;
     const int nch = (M + 4095) / 4096;

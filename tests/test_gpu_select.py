@@ -75,6 +75,23 @@ def test_score_order_sorts_of_two_to_four_thousand(gpu, M, k, gen):
     check_topk(gpu, s, k)
 
 
+@pytest.mark.parametrize("k", [129, 1023, 1025, 2047, 4095, 4097, 8191, 8192])
+@pytest.mark.parametrize("gen", ["smooth", "outlier", "crowd"])
+def test_score_order_bin_sort_edges(gpu, k, gen):
+    """The key-linear bin sort at the edges of its 1, 4 and 8 pairs per thread: a smooth row, one outlier that puts
+    every other pair into few bins, and 40 values one fp32 step apart beside ties (bins past the limit: the other
+    sorts). Exact against the oracle, values too."""
+    rng = np.random.default_rng(k)
+    R, M = 2, 2 * k + 3
+    s = rng.standard_normal((R, M)).astype(np.float32)
+    if gen == "outlier":
+        s[:, 5] = 3e38
+    elif gen == "crowd":
+        s = (np.float32(1.0) + rng.integers(0, 40, size=(R, M)).astype(np.float32) * np.float32(2.0 ** -23))
+        s[:, ::3] += rng.standard_normal((R, s[:, ::3].shape[1])).astype(np.float32)
+    check_topk(gpu, s, k)
+
+
 @pytest.mark.parametrize("M,k,gen", [(32700, 16384, "normal"), (40000, 20000, "normal"), (32768, 32768, "normal"),
                                      (20000, 9000, "ties"), (12000, 10000, "specials"), (10000, 9000, "zeros"),
                                      (300000, 9000, "normal")])
