@@ -196,20 +196,21 @@ def sparse_partitions(BG: int, rows: int, h: int = 1, merged: bool = False) -> i
 
 
 def merged_partitions(BG: int, rows: int, h: int = 1) -> int:
-    """Split-K count of the fused step's attend (partials merged in-kernel by the last partition to arrive). About 256
-    workgroups over the chip, split by rows first (each row read once) and by head groups after (the kernel adds head
-    groups, which read the same rows twice, until the grid reaches 256); at least 128 rows per partition, at most 16
-    partitions, or 8 with four or more heads per KV group, where two head groups also come first from 32 (b, g) rows
-    on (a four-head workgroup's arithmetic then costs more than the second read).
-    Measured on MI355X, step per layer, the rule's P against the best of P in {1, 2, 4, 8, 16, 32}:
-    32K (S = 1092): B=1..2 P=8 best for h = 1, 2, 4; B=4 h=1 P=8 (30.8 us), h=2 P=8 31.79 against P=4 31.45, h=4
-    P=4 (32.8); B=8 P=4 / 4 / 2 best for h = 1 / 2 / 4; B=16 P=2 / 2 / 1 best (h=1 70.39 against 72.14 at P=1).
-    128K (S = 4164): B=1 h=2 P=16 best (40.39), h=4 P=8 40.9 against P=16 40.69; B=2 h=2 P=16 54.57 against P=8
-    54.2, h=4 P=8 best (56.04; 59.58 at P=4); B=4 h=2 P=8 best (93.11), h=4 P=4 best (95.36)."""
+    """Split-K count of the fused step's attend (partials merged in-kernel by the last partition to arrive): one round
+    of at most 256 workgroups (a workgroup of the one-launch select and attend fills a CU), split by rows first and by
+    head groups after (the kernel adds head groups, which read the same rows again, while the grid stays within 256;
+    with four or more heads per KV group two head groups come first, since a four-head workgroup's arithmetic costs
+    more than the second read). At least 128 rows per partition, from 448 rows on up to 8 partitions of 56 rows or more
+    (12K, S = 454: B=2 h=1 17.6 us at P=8 against 18.3 at P=3; a 162-row list loses 1 us to any merge), at most 16
+    partitions (8 with four or more heads per KV group).
+    Measured on MI355X, step per layer, every P in {1, 2, 3, 4, 5, 6, 8, 10, 12, 16} with every head split, the rule
+    against the grids of up to two rounds it replaces: 32K (S = 1092) B=3 h=2 26.6 against 34.1 us, B=5 h=4 38.6 /
+    46.9, B=7 h=2 40.2 / 48.4, B=12 h=1 55.6 / 63.9; 12K (S = 454) B=5 h=4 22.3 / 30.3, B=12 h=2 37.0 / 44.1, B=24
+    h=1 51.4 / 60.4; 3K (S = 162) B=12 h=4 20.6 / 26.7, B=2 h=4 14.5 at P=1 against 15.7 at P=2; B = 1, 2, 16 at 32K
+    as before. The largest miss against the best of all these: 0.8 us (32K, B=12, h=4)."""
     hg = h & -h if h > 0 else 1
-    q = 2 if hg >= 4 and BG >= 32 else 1
-    max_p = 8 if hg >= 4 else 16
-    return auto_partitions(BG * q, rows, max_p=max_p, min_rows=128, blocks=256)
+    by_rows = rows // 128 if rows < 448 else max(8, rows // 128)
+    return max(1, min(8 if hg >= 4 else 16, by_rows, 256 // (max(BG, 1) * (2 if hg >= 4 else 1))))
 
 
 def dense_partitions(BG: int, length: int) -> int:

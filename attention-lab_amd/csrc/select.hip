@@ -1887,10 +1887,20 @@ int select_lists_impl(const float* scores, int64_t score_stride, int B, int G, i
     return check_launch("select_lists");
 }
 
+// Head groups of the one-launch select and attend: as many as keep the grid within one workgroup per CU. A workgroup
+// fills a CU (its LDS), so one more than 256 costs a second round with its whole selection: at 12K, B=5, h=4 (P = 3) two
+// head groups (240 workgroups) take 22.3 us per layer against 30.3 for four (480); at 32K, B=3, h=2 (P = 8) one (192)
+// takes 26.6 against 34.1 for two (384).
+static int fused_head_groups(int BG, int h, int P) {
+    int Q = 1;
+    while (h % (2 * Q) == 0 && (int64_t)BG * P * 2 * Q <= 256) Q *= 2;
+    return Q;
+}
+
 bool select_attend_applies(int B, int G, int lo, int hi, int legal, int k, int h, int P) {
     if (k <= 0 || hi - lo > kListMaxM || P < 1 || h < 1) return false;
     const int S = lo + (legal - hi) + k;
-    const int Q = attend_head_groups(B * G, h, P);
+    const int Q = fused_head_groups(B * G, h, P);
     const int hq = h / Q;
     return (hq == 1 || hq == 2 || hq == 4) && (S + P - 1) / P <= kSAMaxRows && Q <= kSAReadCounter - kArriveOffset;
 }
@@ -1907,7 +1917,7 @@ int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, ui
                   state};
     ListArgs t{lists.entries, lists.hdr, lists.cap, geo.tiles, geo.nsub,
                list_lspl(geo.tiles, kSAWaves, kSASlots, lists.lmin), table};
-    const int Q = attend_head_groups(B * G, h, P);
+    const int Q = fused_head_groups(B * G, h, P);
     AttendArgs a{K, V, (int64_t)C * kHeadDim, kHeadDim, q, nullptr, 0, S, C, h, P, Q, scale * kLog2e, out, 1, part};
     if (P > 1) {
         a.arrive = state + kArriveOffset;

@@ -25,3 +25,14 @@ def test_short_lists_are_not_split_below_128_rows_and_the_combine_rule_is_unchan
     assert merged_partitions(8, 132, 2) == 1 and merged_partitions(8, 300, 2) == 2
     # the standalone attend (combine kernel): B=1 P=8, B=16 h=4 P=1 (two head groups), B=16 h=1 P=1
     assert sparse_partitions(8, 1092, 2) == 8 and sparse_partitions(128, 1092, 4) == 1 and sparse_partitions(128, 1092, 1) == 1
+
+
+@pytest.mark.parametrize("h", [1, 2, 4, 8])
+def test_merged_rule_never_asks_for_a_second_round(h):
+    """Every batch and row count: at most 256 workgroups (one round, a workgroup fills a CU) wherever the (b, g) rows
+    alone allow it, and no partition without rows."""
+    for BG in range(1, 300):
+        for S in (1, 68, 127, 132, 300, 447, 448, 454, 1092, 4164, 9000):
+            P = merged_partitions(BG, S, h)
+            assert 1 <= P <= max(1, min(16, S // 56))
+            assert P == 1 or BG * P <= 256
