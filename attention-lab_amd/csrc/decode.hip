@@ -94,8 +94,21 @@ int sparse_decode_step_impl(const uint16_t* q_main, const uint16_t* K, const uin
     // the list select (it needs the select state, and sorts at most kMaxScoreOrderK picks by score): lists in the
     // select scratch region; otherwise the tiled select, whose scratch (sized for score order) holds the radix sort's
     // buffers
-    const ListPlan plan = k > 0 && state && !staged_score_order(order, k) ? list_plan(hi - lo, k, geo) : ListPlan{0, 0};
-    const ScoreLists lists = plan.cap > 0 ? list_layout(ws + L.sel, B * G, geo, plan) : ScoreLists{};
+    ListPlan plan = k > 0 && state && !staged_score_order(order, k) ? list_plan(hi - lo, k, geo) : ListPlan{0, 0};
+    ScoreLists lists = plan.cap > 0 ? list_layout(ws + L.sel, B * G, geo, plan) : ScoreLists{};
+    if (k > 0 && state && hi - lo > kListMaxM && !rows_out && !rows_flat &&
+        select_attend_applies(B, G, lo, hi, legal, k, h, P)) {
+        // a longer row whose list stays in the call: the same two launches (score with lists, select and attend) instead
+        // of score, classify, resolve and attend. No score is stored then, and the lists take the scores' place (they
+        // fit there unless k is a large part of the row), so the workspace keeps its size. k = M / 32, per layer, four
+        // launches against two: 128K B=1 h=2 39.2 / 37.3 us, B=2 h=2 54.9 / 50.9, B=4 h=2 93.1 / 82.3; 64K B=1 h=2 28.7 /
+        // 26.4, B=4 h=4 52.1 / 48.5; 40K B=8 h=2 60.4 / 54.2.
+        const ListPlan lp = list_plan(hi - lo, k, geo, kListLongM);
+        if (lp.cap > 0 && list_bytes(B * G, geo, lp) <= L.rows - L.scores) {
+            plan = lp;
+            lists = list_layout(ws + L.scores, B * G, geo, lp);
+        }
+    }
     // Stored scores are read only by the tiled select and by score order (which reads the picks' scores back to sort
     // them); the list select in position order recomputes the rare tile it needs from the table and u, so the score
     // kernel then writes key lists only.

@@ -272,14 +272,16 @@ FusedGeometry fused_geometry(int BG, int C, int r, int hd, int lo, int hi, const
 // holds at least lmin keys (its even share s of the k plus 3 sqrt(s) + 16, so that a list misses part of the row's
 // selection only when its tile holds several standard deviations more than its share), and at most cap (lmin plus
 // 192, for the keys of the first-digit bin holding the lmin-th key). cap == 0: the list select does not apply (rows
-// past 32768 candidates or 128 tiles, or lists that would hold half a tile or more).
+// past max_m candidates or 128 tiles, or lists that would hold half a tile or more). max_m is kListMaxM where the rows
+// leave the select as a list (select_lists), kListLongM where the one-launch select and attend keeps them.
 constexpr int kListMaxM = 32768;
+constexpr int kListLongM = 131072;
 constexpr int kListMaxTiles = 128;
 struct ListPlan {
     int lmin, cap;
 };
-inline ListPlan list_plan(int M, int k, FusedGeometry g) {
-    if (g.nsub == 0 || k <= 0 || M > kListMaxM || g.tiles > kListMaxTiles) return ListPlan{0, 0};
+inline ListPlan list_plan(int M, int k, FusedGeometry g, int max_m = kListMaxM) {
+    if (g.nsub == 0 || k <= 0 || M > max_m || g.tiles > kListMaxTiles) return ListPlan{0, 0};
     const int nw = 512 * g.nsub;
     const int64_t share = ((int64_t)k * nw + M - 1) / M;
     int64_t root = 0;

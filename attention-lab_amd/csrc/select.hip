@@ -1531,16 +1531,25 @@ constexpr int kSAThreads = 512;
 constexpr int kSAWaves = kSAThreads / 64;
 constexpr int kSASlots = 8;            // list entries per lane in the first round trip
 constexpr int kSAMaxRows = 4096;       // positions of one partition held in LDS
+// Rows past 32768 candidates (to kListLongM) run an instance of their own: four times the bitmap, twice the slots (their
+// lists hold about 230 entries each, four lists a wave; 8 and 32 slots are equal at 128K, 64K loses 1.3 us to either) and
+// partitions of up to 8192 positions. The selection bounds it there: 12.8 us of its 22.7 at 128K, B=2, k = 4096 (first
+// round trip 1.9, the slots 3.5, the lists' tails 3.3, waiting for the slowest wave 1.2, the digits 1.2, the row list
+// 1.7). One LDS atomic per slot for both kinds of keys, the bitmap's words rotated over the LDS banks, and 1024 threads
+// (scratch memory at two heads, 27.8 us) were no faster.
+constexpr int kSALongSlots = 16;
+constexpr int kSALongMaxRows = 8192;
 // K/V register stages of the fused attend (attend_kernel keeps kStages): the output does not depend on the depth, and
 // three measured 0.08-0.14 us per layer faster than four at B = 1, 2, 4, 8 and 16 (two: up to 3 us slower)
 constexpr int kSAStages = 3;
 constexpr int kSAReadCounter = kSelectStateWords - 1;   // the row's readers of its bins: the last arrival word
 static_assert(kListWords == 2 * kSAThreads, "two selection bitmap words per thread");
 
-template <int MAXSUB, int H>
+template <int MAXSUB, int H, int WORDS = kListWords, int SLOTS = kSASlots>
 __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListArgs t, AttendArgs a) {
+    constexpr int kWPT = WORDS / (2 * kSAThreads);   // 64-bit bitmap words per thread
     __shared__ __attribute__((aligned(16))) uint32_t hist[kHistBins];
-    __shared__ __attribute__((aligned(16))) uint32_t lds[2048 + 1024 + 2 * kListWords];
+    __shared__ __attribute__((aligned(16))) uint32_t lds[2048 + 1024 + 2 * WORDS];
     __shared__ __attribute__((aligned(16))) uint2 cand[kListCandCap];
     __shared__ uint2 hdr[kListMaxTiles];
     __shared__ uint32_t sup2[64];
@@ -1550,7 +1559,7 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     __shared__ __attribute__((aligned(16))) float red_acc[kMergeSlots][H][kHeadDim];
     __shared__ uint32_t last_sh;
     int* idx_sh = reinterpret_cast<int*>(cand);   // the partition's positions, once the selection no longer needs cand
-    static_assert(kSAMaxRows * sizeof(int) <= sizeof(cand), "the positions fit the candidate array");
+    static_assert(kSALongMaxRows * sizeof(int) <= sizeof(cand), "the positions fit the candidate array");
     const int lin = xcd_contiguous_block();   // (b, g) on the XCD whose score workgroups wrote its lists
     const int bg = lin / (a.Q * a.P);
     const int rem = lin - bg * a.Q * a.P;
@@ -1569,7 +1578,7 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     L.sup2 = sup2;
     L.hist3 = lds + 2048;
     L.bits = lds + 3072;
-    L.ties = lds + 3072 + kListWords;
+    L.ties = lds + 3072 + WORDS;
     L.hdr = hdr;
     L.cand = cand;
     L.misc = misc;
@@ -1587,32 +1596,42 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     r.tiles = t.tiles;
     r.nsub = t.nsub;
     r.lspl = t.lspl;
-    list_select_bitmap<kSAThreads, kSASlots, MAXSUB>(r, L);
-    // this thread's selected candidates [64 tid, 64 tid + 64) and their first slot among the k picks
-    const uint2 wv = reinterpret_cast<const uint2*>(L.bits)[tid];
-    uint64_t word = (uint64_t)wv.x | ((uint64_t)wv.y << 32);
-    const uint32_t x = (uint32_t)__popcll(word);
+    list_select_bitmap<kSAThreads, SLOTS, MAXSUB, WORDS>(r, L);
+    // this thread's selected candidates [64 kWPT tid, 64 kWPT (tid + 1)) and their first slot among the k picks
+    uint64_t words[kWPT];
+    uint32_t x = 0u;
+#pragma unroll
+    for (int i = 0; i < kWPT; ++i) {
+        const uint2 wv = reinterpret_cast<const uint2*>(L.bits)[kWPT * tid + i];
+        words[i] = (uint64_t)wv.x | ((uint64_t)wv.y << 32);
+        x += (uint32_t)__popcll(words[i]);
+    }
     const uint32_t inc = wave_incl_scan(x);
     if (lane == 63) wave_tot[wave][0] = inc;
     __syncthreads();   // also: the candidates (cand) are no longer read, so idx_sh may take their place
     const uint32_t v = lane < kSAWaves ? wave_tot[lane][0] : 0u;
     const uint32_t vi = row16_incl_scan(v);
-    const uint32_t slot = (uint32_t)__builtin_amdgcn_readlane((int)(vi - v), wave) + inc - x;
+    int slot = (int)((uint32_t)__builtin_amdgcn_readlane((int)(vi - v), wave) + inc - x);
     // the partition's entries of the row list [F sinks | the k picks by position | F recent]
     const int lo = sa.lo, k = sa.k, nrec = sa.legal - sa.hi, nf = lo + nrec;
     const int Sp = (a.S + a.P - 1) / a.P;
     const int s_begin = p * Sp, s_end = min(a.S, s_begin + Sp);
-    const int pos0 = lo + 64 * tid;
-    // this thread's picks take slots [slot, slot + x) of the k (row-list entries lo + slot ..); those inside the
+    // a word's picks take slots [slot, slot + its bits) of the k (row-list entries lo + slot ..); those inside the
     // partition, [first, last), go to LDS: the picks before it are dropped, and no lane loops over picks past it
-    const int first = max((int)slot, s_begin - lo), last = min((int)slot + (int)x, min(s_end - lo, k));
-    if (first < last) {
-        for (int j = (int)slot; j < first; ++j) word &= word - 1;
-        int* dst = idx_sh + (lo + first - s_begin);
-        for (int n = last - first; n > 0; --n) {
-            *dst++ = pos0 + (__ffsll((unsigned long long)word) - 1);
-            word &= word - 1;
+#pragma unroll
+    for (int i = 0; i < kWPT; ++i) {
+        uint64_t word = words[i];
+        const int pos0 = lo + 64 * (kWPT * tid + i), n = (int)__popcll(word);
+        const int first = max(slot, s_begin - lo), last = min(slot + n, min(s_end - lo, k));
+        if (first < last) {
+            for (int j = slot; j < first; ++j) word &= word - 1;
+            int* dst = idx_sh + (lo + first - s_begin);
+            for (int m = last - first; m > 0; --m) {
+                *dst++ = pos0 + (__ffsll((unsigned long long)word) - 1);
+                word &= word - 1;
+            }
         }
+        slot += n;
     }
     for (int f = tid; f < nf; f += kSAThreads) {
         const int e = f < lo ? f : lo + k + (f - lo);
@@ -1898,11 +1917,12 @@ static int fused_head_groups(int BG, int h, int P) {
 }
 
 bool select_attend_applies(int B, int G, int lo, int hi, int legal, int k, int h, int P) {
-    if (k <= 0 || hi - lo > kListMaxM || P < 1 || h < 1) return false;
+    if (k <= 0 || hi - lo > kListLongM || P < 1 || h < 1) return false;
     const int S = lo + (legal - hi) + k;
+    const int max_rows = hi - lo > kListMaxM ? kSALongMaxRows : kSAMaxRows;
     const int Q = fused_head_groups(B * G, h, P);
     const int hq = h / Q;
-    return (hq == 1 || hq == 2 || hq == 4) && (S + P - 1) / P <= kSAMaxRows && Q <= kSAReadCounter - kArriveOffset;
+    return (hq == 1 || hq == 2 || hq == 4) && (S + P - 1) / P <= max_rows && Q <= kSAReadCounter - kArriveOffset;
 }
 
 int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, uint32_t* state, const ScoreLists& lists,
@@ -1916,7 +1936,7 @@ int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, ui
     SelectArgs sa{nullptr, 0, M, k, lo, hi, legal, G, C, ATTNLAB_ORDER_POSITION, nullptr, 0, nullptr, nullptr, nullptr, 0,
                   state};
     ListArgs t{lists.entries, lists.hdr, lists.cap, geo.tiles, geo.nsub,
-               list_lspl(geo.tiles, kSAWaves, kSASlots, lists.lmin), table};
+               list_lspl(geo.tiles, kSAWaves, M > kListMaxM ? kSALongSlots : kSASlots, lists.lmin), table};
     const int Q = fused_head_groups(B * G, h, P);
     AttendArgs a{K, V, (int64_t)C * kHeadDim, kHeadDim, q, nullptr, 0, S, C, h, P, Q, scale * kLog2e, out, 1, part};
     if (P > 1) {
@@ -1931,7 +1951,11 @@ int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, ui
         else if (hq == 2) hipLaunchKernelGGL((select_attend<MS, 2>), grid, block, 0, stream, sa, t, a);   \
         else hipLaunchKernelGGL((select_attend<MS, 4>), grid, block, 0, stream, sa, t, a);                \
     } while (0)
-    if (geo.nsub <= 4) SA_LAUNCH(4);
+    if (M > kListMaxM) {
+        if (hq == 1) hipLaunchKernelGGL((select_attend<8, 1, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
+        else if (hq == 2) hipLaunchKernelGGL((select_attend<8, 2, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
+        else hipLaunchKernelGGL((select_attend<8, 4, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
+    } else if (geo.nsub <= 4) SA_LAUNCH(4);
     else SA_LAUNCH(8);
 #undef SA_LAUNCH
     return check_launch("select_attend");

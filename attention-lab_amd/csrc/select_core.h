@@ -1,5 +1,5 @@
 // The list select of one row as a device function (select_lists runs it with 1024 threads per row; the code takes
-// any multiple of 64 threads up to 1024 that divides the 1024-word bitmap).
+// any multiple of 64 threads up to 1024 that divides the bitmap's WORDS words: 1024, or 4096 for rows past 32768).
 //
 // The score kernel leaves, per workgroup of a row, a list of its largest keys (every key whose first digit is at least
 // that of the workgroup's lmin-th largest, d_L) with a header (d_L, length). list_select_bitmap then
@@ -26,6 +26,7 @@ namespace attnlab {
 
 constexpr int kListCandCap = 8192;                    // keys of bin b1 held in LDS as (index, low 21 key bits)
 constexpr int kListWords = kListMaxM / 32;            // selection bitmap words: 1024
+constexpr int kListLongWords = kListLongM / 32;       // of the longer rows' instance: 4096
 
 // One row of the list select. The score kernel's tiling (nsub sub-tiles of 512 columns per workgroup, tiles
 // workgroups) locates an incomplete list's scores.
@@ -46,8 +47,8 @@ struct ListLds {
     uint32_t* hist2;          // 2048: the second digit over bin b1
     uint32_t* sup2;           // 64: super-bins of hist2
     uint32_t* hist3;          // 1024: the third digit
-    uint32_t* bits;           // kListWords: the selection bitmap (the result)
-    uint32_t* ties;           // kListWords
+    uint32_t* bits;           // WORDS: the selection bitmap (the result)
+    uint32_t* ties;           // WORDS
     uint2* hdr;               // kListMaxTiles
     uint2* cand;              // kListCandCap
     uint32_t* misc;           // 4: candidate count, then a wave-0 search's digit, keys left, bin count
@@ -143,9 +144,9 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t& total,
 }
 
 // The first krem tied keys in index order join the selection: thread t owns words [t W, t W + W) of both bitmaps.
-template <int THREADS>
+template <int THREADS, int WORDS>
 __device__ __forceinline__ void take_ties(const ListLds& L, uint32_t krem) {
-    constexpr int W = kListWords / THREADS;
+    constexpr int W = WORDS / THREADS;
     const int tid = threadIdx.x;
     uint32_t n = 0;
 #pragma unroll
@@ -170,7 +171,7 @@ __device__ __forceinline__ void take_ties(const ListLds& L, uint32_t krem) {
 // passes are one loop (pass 0: second digit of bin b1's keys; pass 1: third digit of prefix p2; pass 2: keys above
 // and equal to the threshold T into the two bitmaps), so the score read, possibly a recompute from the table, is
 // emitted once.
-template <int THREADS>
+template <int THREADS, int WORDS>
 __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L, uint32_t b1, uint32_t krem) {
     const int tid = threadIdx.x;
     uint32_t prefix = b1;   // pass 0: the first digit; pass 1: the first two (p2); pass 2: the threshold key T
@@ -205,18 +206,18 @@ __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L,
         }
         krem = pass < 2 ? L.misc[2] : krem;
     }
-    take_ties<THREADS>(L, krem);
+    take_ties<THREADS, WORDS>(L, krem);
 }
 
 // The selection bitmap of one row (in L.bits, complete and synchronised on return). SLOTS: entries per lane loaded
 // in the first round trip (the first 64 << r.lspl entries of each of the wave's first SLOTS >> r.lspl lists; later
 // entries and lists are read afterwards). MAXSUB (4 or 8): the most sub-tiles per score workgroup this instance reads
 // for an incomplete list (r.nsub <= MAXSUB). Called by every thread of the workgroup.
-template <int THREADS, int SLOTS, int MAXSUB>
+template <int THREADS, int SLOTS, int MAXSUB, int WORDS = kListWords>
 __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListLds& L) {
     static_assert(MAXSUB == 4 || MAXSUB == 8, "sub-tiles are read four at a time");
     constexpr int kWaves = THREADS / 64;
-    constexpr int W = kListWords / THREADS;
+    constexpr int W = WORDS / THREADS;
     static_assert(SLOTS % 8 == 0, "slots are taken in passes of 8");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nt = r.tiles;
@@ -259,7 +260,7 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
     const uint32_t b1 = wave_first_digit(sbv, L.hist, (uint32_t)r.k, above, nb1);
     uint32_t krem = (uint32_t)r.k - above;
     if (nb1 > (uint32_t)kListCandCap) {   // the same test in every wave
-        radix_bitmap<THREADS>(r, L, b1, krem);
+        radix_bitmap<THREADS, WORDS>(r, L, b1, krem);
         return;
     }
     const uint32_t M = (uint32_t)r.M;
@@ -443,7 +444,7 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
         else if (c.y == tlow) atomicOr(&L.ties[c.x >> 5], 1u << (c.x & 31u));
     }
     __syncthreads();
-    take_ties<THREADS>(L, krem);
+    take_ties<THREADS, WORDS>(L, krem);
 }
 
 }  // namespace attnlab

@@ -671,3 +671,21 @@ def test_fused_select_attend_equals_the_separate_stages(gpu, B, G, h, C, L, rho,
     s = kernel_scores(zT, q_pre, idx, lo, hi)
     want = exact.select_rows(s, lo, hi, L, req.k, order="position")
     check_out(outs[0], exact.subset_attention(f64(q)[:, :, :, 0], f64(K), f64(V), want), f"{case} P={P}")
+
+
+@pytest.mark.parametrize("B,G,h,L,rho,case,P", [
+    (1, 2, 2, 32768 + 69, 1 / 32, None, None),          # one candidate past the shorter instance's bitmap
+    (1, 8, 1, 40003, 1 / 32, None, None),
+    (2, 3, 4, 131072 + 68, 1 / 32, None, None),         # the longest row: every word of its bitmap
+    (1, 2, 2, 131072 + 69, 1 / 32, None, None),         # one past it: the separate launches on both sides
+    (1, 2, 8, 65536, 1 / 64, None, 3),                  # odd partitions, four heads per workgroup
+    (1, 1, 2, 131000, 1 / 16, None, 1),                 # one partition of 8254 rows: not taken
+    (1, 2, 2, 100001, 1 / 32, "all_equal", None),
+    (1, 2, 2, 100001, 1 / 32, "skewed_tile", 2),
+    (2, 2, 1, 70000, 1 / 32, "seven_values", None),
+])
+def test_fused_select_attend_on_rows_past_32768(gpu, B, G, h, L, rho, case, P):
+    """The longer rows' instance (a 4096-word bitmap, the lists in the scores' place) against the tiled select and the
+    separate attend, bit for bit, and the float64 oracle; the score distributions that leave lists incomplete or crowd
+    the threshold's bin take the recomputed tiles and the radix passes."""
+    test_fused_select_attend_equals_the_separate_stages(gpu, B, G, h, -(-L // 8) * 8, L, rho, case, P)
