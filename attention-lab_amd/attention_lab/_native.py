@@ -8,6 +8,7 @@ cannot load, every op raises RuntimeError.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -118,8 +119,16 @@ def call(name: str, *args) -> None:
 
 
 def stream_of(device: torch.device) -> int:
-    """hipStream_t of torch's current stream on `device` (kernels launch where torch would launch)."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on `device` (kernels launch where torch would launch). The raw handle:
+    building torch's Stream object around it cost 4 us of a call's 22."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+
+
+@functools.lru_cache(maxsize=1024)
+def step_workspace_bytes(B: int, G: int, h: int, lo: int, hi: int, legal: int, k: int, P: int) -> int:
+    """attnlab_sparse_decode_workspace, a function of the sizes alone (every layer of a step asks for the same ones)."""
+    return lib().attnlab_sparse_decode_workspace(B, G, h, lo, hi, legal, k, P)
 
 
 def ptr(t) -> int | None:

@@ -27,7 +27,7 @@ from . import _native as nat
 from . import hip_attend, hip_score, hip_select
 from .indexer import GroupedIndexer
 from .selection import FIXED_PREFIX, FIXED_RECENT, SelectionLayout, fixed_budget, legal_length, selection_layout
-from .sparse import flatten_cache, row_offsets
+from .sparse import check_flat, row_offsets
 
 SUBSET_BACKENDS = ("sdpa", "explicit")
 
@@ -199,8 +199,8 @@ def gathered_decode_step_kernel(q_main, k_cache, v_cache, rows, selected_count: 
     B, G, h, T, d = q_main.shape
     if T != 1:
         raise ValueError("a decode step takes exactly one new query position")
-    flatten_cache(k_cache)
-    flatten_cache(v_cache)
+    check_flat(k_cache)
+    check_flat(v_cache)
     C = int(k_cache.shape[2])
     pos = _positions_from_flat(rows, B, G, selected_count, C, k_cache.device)
     q = q_main.reshape(B, G, h, d).contiguous()
@@ -231,17 +231,20 @@ def sparse_decode_step_kernel(q_main, q_pre, k_cache, v_cache, zT, wq_t_scaled, 
     idx_dt = zT.dtype
     if idx_dt not in (torch.bfloat16, torch.float32):
         raise ValueError(f"zT must be bfloat16 or float32, got {idx_dt}")
-    for t, n, want in ((q_main, "q_main", torch.bfloat16), (q_pre, "q_pre", idx_dt), (k_cache, "k_cache", torch.bfloat16),
-                       (v_cache, "v_cache", torch.bfloat16), (zT, "zT", idx_dt), (wq_t_scaled, "wq_t_scaled", idx_dt),
-                       (wk, "wk", idx_dt)):
-        if t.dtype != want:
-            raise ValueError(f"{n} must be {want} on the HIP path, got {t.dtype}")
-        if not t.is_cuda:
-            raise ValueError(f"{n} must live on a HIP device")
+    if not (q_main.dtype == k_cache.dtype == v_cache.dtype == torch.bfloat16
+            and q_pre.dtype == wq_t_scaled.dtype == wk.dtype == idx_dt and q_main.is_cuda and q_pre.is_cuda
+            and k_cache.is_cuda and v_cache.is_cuda and zT.is_cuda and wq_t_scaled.is_cuda and wk.is_cuda):
+        for t, n, want in ((q_main, "q_main", torch.bfloat16), (q_pre, "q_pre", idx_dt),
+                           (k_cache, "k_cache", torch.bfloat16), (v_cache, "v_cache", torch.bfloat16),
+                           (zT, "zT", idx_dt), (wq_t_scaled, "wq_t_scaled", idx_dt), (wk, "wk", idx_dt)):
+            if t.dtype != want:
+                raise ValueError(f"{n} must be {want} on the HIP path, got {t.dtype}")
+            if not t.is_cuda:
+                raise ValueError(f"{n} must live on a HIP device")
     if d != hip_attend.HEAD_DIM or not 1 <= h <= hip_attend.MAX_H:
         raise ValueError(f"the HIP path needs head_dim {hip_attend.HEAD_DIM} and 1 <= h <= {hip_attend.MAX_H}")
-    flatten_cache(k_cache)
-    flatten_cache(v_cache)
+    check_flat(k_cache)
+    check_flat(v_cache)
     Bc, Gc, C, dc = k_cache.shape
     if (Bc, Gc, dc) != (B, G, d) or v_cache.shape != k_cache.shape:
         raise ValueError("k_cache/v_cache must be [B, G, C, d] matching q_main")
@@ -257,13 +260,18 @@ def sparse_decode_step_kernel(q_main, q_pre, k_cache, v_cache, zT, wq_t_scaled, 
     if legal > C:
         raise ValueError(f"legal length {legal} exceeds capacity {C}")
     check_standard_f(fixed_rows, off_lo, lo, hi, legal, C)
-    q = q_main.reshape(B, G, h, d).contiguous()
-    q_cat = q_pre.reshape(B, G, h * d).contiguous()
+    # operands whose elements already lie in the kernels' order are passed as they are: a reshape of a contiguous tensor
+    # is the same memory, and a view object costs more than a microsecond
+    q = q_main if q_main.is_contiguous() else q_main.reshape(B, G, h, d).contiguous()
+    if q_pre.is_contiguous() and q_pre.numel() == q_main.numel():
+        q_cat = q_pre
+    else:
+        q_cat = q_pre.reshape(B, G, h * d).contiguous()
     k_new = None
     if k_pre_new is not None:
         if tuple(k_pre_new.shape) != (B, G, 1, d) or k_pre_new.dtype != idx_dt:
             raise ValueError(f"k_pre_new must be a {idx_dt} [B, G, 1, d] tensor")
-        k_new = k_pre_new.reshape(B, G, d).contiguous()
+        k_new = k_pre_new if k_pre_new.is_contiguous() else k_pre_new.reshape(B, G, d).contiguous()
         wc = int(write_col) if write_col >= 0 else C + int(write_col)
         if not 0 <= wc < C or lo <= wc < hi:
             raise ValueError(f"write_col={write_col} must lie in [0, C) and outside [lo, hi)")
@@ -272,12 +280,13 @@ def sparse_decode_step_kernel(q_main, q_pre, k_cache, v_cache, zT, wq_t_scaled, 
     P = hip_attend.sparse_partitions(B * G, S, h, merged=k > 0) if partitions is None else int(partitions)
     sc = float(1.0 / math.sqrt(d) if scale is None else scale)
     order = nat.ORDER_POSITION if canonical_order else nat.ORDER_SCORE
-    nbytes = nat.lib().attnlab_sparse_decode_workspace(B, G, h, lo, hi, legal, k, P)
+    nbytes = nat.step_workspace_bytes(B, G, h, lo, hi, legal, k, P)
     wsp = _STEP_WS if workspace is None else workspace
     ws = wsp.bytes(k_cache.device, nbytes, "step")
     # select state: zeroed once, left zeroed by each call
     state = wsp.bytes(k_cache.device, B * G * nat.SELECT_STATE_WORDS * 4, "state")
-    out = torch.empty(B, G, h, d, dtype=torch.bfloat16, device=k_cache.device)
+    device = k_cache.device
+    out = torch.empty(B, G, h, 1, d, dtype=torch.bfloat16, device=device)
     flat = torch.empty(B * G * S, dtype=torch.int64, device=k_cache.device) if return_rows else None
     entry = "attnlab_sparse_decode_step" if idx_dt == torch.bfloat16 else "attnlab_sparse_decode_step_f32"
     # contiguous copies (if any) are held here: a temporary's memory could go to the next one before the launch
@@ -285,8 +294,7 @@ def sparse_decode_step_kernel(q_main, q_pre, k_cache, v_cache, zT, wq_t_scaled, 
     nat.call(entry, q.data_ptr(), q_cat.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
              zT.data_ptr(), wq_c.data_ptr(), wk_c.data_ptr(), nat.ptr(k_new), B, G, h, r,
              C, lo, hi, legal, k, wc, sc, order, P, state.data_ptr(), ws.data_ptr(), ws.numel(), None, nat.ptr(flat),
-             out.data_ptr(), nat.stream_of(k_cache.device))
-    out = out.view(B, G, h, 1, d)
+             out.data_ptr(), nat.stream_of(device))
     return (out, flat) if return_rows else out
 
 

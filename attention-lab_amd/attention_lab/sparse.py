@@ -18,12 +18,17 @@ def row_offsets(batch: int, groups: int, capacity: int, device) -> torch.Tensor:
     return (torch.arange(batch * groups, device=device, dtype=torch.long) * capacity).view(batch, groups, 1)
 
 
-def flatten_cache(x: torch.Tensor) -> torch.Tensor:
-    """[B,G,C,d] contiguous -> [B*G*C, d] view. Never copies: raises instead."""
+def check_flat(x: torch.Tensor) -> None:
+    """flatten_cache's checks alone, for callers that hand the cache's address on and need no view."""
     if x.dim() != 4:
         raise ValueError(f"cache must be [B,G,C,d], got {tuple(x.shape)}")
     if not x.is_contiguous():
         raise ValueError("cache must be contiguous so the flattened view is free")
+
+
+def flatten_cache(x: torch.Tensor) -> torch.Tensor:
+    """[B,G,C,d] contiguous -> [B*G*C, d] view. Never copies: raises instead."""
+    check_flat(x)
     B, G, C, d = x.shape
     return x.view(B * G * C, d)
 
