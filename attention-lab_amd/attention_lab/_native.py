@@ -17,7 +17,7 @@ import torch
 LIB_NAME = "libattnlab.so"
 # ATTNLAB_LIB names another build of the same library (the host-sanitized debug build); unset, the in-tree one
 LIB_PATH = os.environ.get("ATTNLAB_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 9
+ABI_VERSION = 10
 # select state per (b, g) row: the first-digit histogram of the top-k (2048 bins, top 11 bits of the order-preserving
 # score key), 64 super-bin counts of 32 bins each, then 64 arrival counters of the step's attend partitions
 # (ATTNLAB_SELECT_STATE_WORDS)
@@ -44,6 +44,8 @@ SIGNATURES = {
     "attnlab_score_lightning_batched": (_i, [_p, _i, _p, _p, _p, _i64] + [_i] * 10 + [_p]),
     "attnlab_topk": (_i, [_p, _i64] + [_i] * 4 + [_p, _p, _i64, _p]),
     "attnlab_topk_tiled": (_i, [_p, _i64] + [_i] * 4 + [_p, _p, _i64, _p, _p, _i64, _p]),
+    "attnlab_topk_i64": (_i, [_p, _i64] + [_i] * 4 + [_p, _p, _p]),
+    "attnlab_topk_tiled_i64": (_i, [_p, _i64] + [_i] * 4 + [_p, _p, _p, _p, _i64, _p]),
     "attnlab_select_rows": (_i, [_p, _i64] + [_i] * 8 + [_p, _i64, _p, _p, _p, _i64, _p]),
     "attnlab_select_scratch_bytes": (_i64, [_i] * 4),
     "attnlab_list_bytes": (_i64, [_i] * 6),

@@ -17,7 +17,7 @@ import torch
 from . import _native as nat
 
 LDS_SORT_K = nat.LDS_SORT_K   # score order up to this k is sorted in LDS; past it, by a radix pass (tiled entry)
-TILED_MIN_M = 32768     # rows at least this long are selected by the tiled kernels (attnlab_topk_tiled)
+TILED_MIN_M = 32768     # rows at least this long are selected by the tiled kernels (attnlab_topk_tiled_i64)
 TILED_MAX_M = 262144    # ... and at most this long (longer rows take the single-workgroup select)
 REG_MAX_M = 32768       # rows up to this long fit the single-workgroup select's registers ...
 REG_MIN_ROWS = 128      # ... which beats the tiled kernels from this many rows on (the rows alone fill half the chip)
@@ -61,7 +61,7 @@ def topk(scores, k: int, *, order: str = "score", tiled=None, workspace=None):
     if s2.stride(-1) != 1:
         s2 = s2.contiguous()
     R = s2.shape[0]
-    idx = torch.empty(R, max(k, 1), dtype=torch.int32, device=scores.device)
+    idx = torch.empty(R, max(k, 1), dtype=torch.int64, device=scores.device)   # written as int64 by the kernels
     val = torch.empty(R, max(k, 1), dtype=torch.float32, device=scores.device)
     if tiled is None:
         tiled = use_tiled(R, M)
@@ -72,12 +72,12 @@ def topk(scores, k: int, *, order: str = "score", tiled=None, workspace=None):
         state = ws.bytes(scores.device, R * nat.SELECT_STATE_WORDS * 4, "state")
         nbytes = nat.lib().attnlab_select_scratch_bytes(R, M, k, code)
         scratch = ws.bytes(scores.device, nbytes, "scratch")
-        nat.call("attnlab_topk_tiled", s2.data_ptr(), s2.stride(0), R, M, k, code, idx.data_ptr(), val.data_ptr(),
-                 idx.stride(0), state.data_ptr(), scratch.data_ptr(), scratch.numel(), nat.stream_of(scores.device))
+        nat.call("attnlab_topk_tiled_i64", s2.data_ptr(), s2.stride(0), R, M, k, code, idx.data_ptr(), val.data_ptr(),
+                 state.data_ptr(), scratch.data_ptr(), scratch.numel(), nat.stream_of(scores.device))
     elif R and k:
-        nat.call("attnlab_topk", s2.data_ptr(), s2.stride(0), R, M, k, code, idx.data_ptr(), val.data_ptr(),
-                 idx.stride(0), nat.stream_of(scores.device))
-    return val[:, :k].reshape(*lead, k), idx[:, :k].long().reshape(*lead, k)
+        nat.call("attnlab_topk_i64", s2.data_ptr(), s2.stride(0), R, M, k, code, idx.data_ptr(), val.data_ptr(),
+                 nat.stream_of(scores.device))
+    return val[:, :k].reshape(*lead, k), idx[:, :k].reshape(*lead, k)
 
 
 def select_rows(scores, lo: int, hi: int, legal: int, k: int, capacity: int, *, order: str = "position",

@@ -513,6 +513,15 @@ __device__ __forceinline__ const uint64_t* radix_sort_desc_4096(SelectShared& sh
     return base + 4096 * cur;
 }
 
+// A top-k with values in position order writes its picks by way of sortbuf (score bits, index) in slot order, like score
+// order: a thread's own picks are a few elements of two output rows, written a lane at a time, and the partly written
+// lines bound the launch where many are picked. int64 indices, written from the emitting thread / by way of LDS: 256 rows
+// of 16K scores, k = 8192, 65.4 / 20.9 us; 256 of 128K, k = 4096, 85.9 / 79.0; 8 of 128K, k = 4096, 23.8 / 22.6; 8 of 4K,
+// k = 256, 7.1 / 6.8; 1 of 4K, k = 128, 6.1 / 6.1. Past sortbuf's 8192 pairs the emitting thread writes.
+__device__ __forceinline__ bool stages_positions(const SelectArgs& a) {
+    return a.order == ATTNLAB_ORDER_POSITION && a.top_val && a.k <= kMaxScoreOrderK;
+}
+
 // F positions and, in score order, the sorted candidates (the selected pairs are staged in sh.sortbuf).
 __device__ __forceinline__ void finish_row(const SelectArgs& a, int row, SelectShared& sh) {
     const int tid = threadIdx.x;
@@ -530,6 +539,19 @@ __device__ __forceinline__ void finish_row(const SelectArgs& a, int row, SelectS
             if (rows) rows[s_out] = pos;
             if (flat) flat[s_out] = base + pos;
         }
+    }
+    if (stages_positions(a)) {
+        __syncthreads();
+        int32_t* ti = a.top_idx ? a.top_idx + (size_t)row * a.top_stride : nullptr;
+        float* tv = a.top_val + (size_t)row * a.top_stride;
+        for (int j = tid; j < k; j += kSelThreads) {
+            const uint64_t e = sh.sortbuf[j];
+            const int idx = min((int)(uint32_t)e, a.M - 1);   // in range for any slot left unwritten
+            if (ti) ti[j] = idx;
+            tv[j] = __uint_as_float((uint32_t)(e >> 32));
+            if (flat) flat[lo + j] = base + lo + idx;
+        }
+        return;
     }
     if (order != ATTNLAB_ORDER_SCORE || k == 0) return;
     // descending on (key, ~index): larger score first, then lower index (sortbuf[0, sort_len(k)) was pre-filled by
@@ -569,6 +591,7 @@ __device__ __forceinline__ void finish_row(const SelectArgs& a, int row, SelectS
 // to the scores can then only give a wrong selection, never a write outside the k output slots.
 struct Emitter {
     int order, lo;
+    bool staged;         // position order by way of sortbuf (stages_positions)
     uint32_t k;
     int32_t* ti;
     float* tv;
@@ -583,6 +606,10 @@ struct Emitter {
         if (slot >= k) return;
         if (order == ATTNLAB_ORDER_SCORE) {
             sortbuf[slot] = ((uint64_t)score_key(v) << 32) | (uint64_t)(0xffffffffu - (uint32_t)idx);
+            return;
+        }
+        if (staged) {
+            sortbuf[slot] = ((uint64_t)__float_as_uint(v) << 32) | (uint32_t)idx;
             return;
         }
         if (ti) ti[slot] = idx;
@@ -626,6 +653,7 @@ __device__ __forceinline__ uint32_t lowest_bits(uint32_t w, uint32_t n) {
 __device__ __forceinline__ Emitter make_emitter(const SelectArgs& a, int row, SelectShared& sh) {
     Emitter e;
     e.order = a.order;
+    e.staged = stages_positions(a);
     e.lo = a.lo;
     e.k = (uint32_t)a.k;
     e.ti = a.top_idx ? a.top_idx + (size_t)row * a.top_stride : nullptr;
@@ -1988,8 +2016,14 @@ int select_rows_impl(const float* scores, int64_t score_stride, int B, int G, in
 
 using namespace attnlab;
 
-extern "C" int attnlab_topk(const float* scores, int64_t score_stride, int R, int M, int k, int order, int32_t* top_idx,
-                            float* top_val, int64_t top_stride, void* stream) {
+namespace {
+
+// The outputs of a standalone top-k: int32 indices beside the values, or (idx64) int64 indices with rows of k, which the
+// kernels write as the flat row ids of a read without a fixed set (lo = hi = legal = C = 0). The caller that wants int64
+// then needs no conversion launch: top-k of 8 rows of 128K scores, k = 4096, 35.5 -> 32.5 us in a replayed graph; 8 rows
+// of 4K, k = 256, 13.2 -> 10.0.
+int topk_impl(const float* scores, int64_t score_stride, int R, int M, int k, int order, int32_t* top_idx, int64_t* idx64,
+              float* top_val, int64_t top_stride, void* stream) {
     ATTNLAB_REQUIRE(R >= 0 && M >= 0, "R=%d and M=%d must be non-negative", R, M);
     ATTNLAB_REQUIRE(0 <= k && k <= M, "need 0 <= k <= M, got k=%d M=%d", k, M);
     ATTNLAB_REQUIRE(order == ATTNLAB_ORDER_POSITION || order == ATTNLAB_ORDER_SCORE, "unknown order %d", order);
@@ -1998,14 +2032,14 @@ extern "C" int attnlab_topk(const float* scores, int64_t score_stride, int R, in
     if (R == 0 || k == 0) return ATTNLAB_OK;
     ATTNLAB_REQUIRE(scores != nullptr && score_stride >= M, "scores must hold M=%d values per row", M);
     ATTNLAB_REQUIRE(top_stride >= k, "top_stride=%lld smaller than k=%d", (long long)top_stride, k);
-    SelectArgs a{scores, score_stride, M, k, 0, 0, 0, 1, 0, order, nullptr, 0, nullptr, top_idx, top_val, top_stride,
+    SelectArgs a{scores, score_stride, M, k, 0, 0, 0, 1, 0, order, nullptr, 0, idx64, top_idx, top_val, top_stride,
                  nullptr};
     return launch_select(a, R, reinterpret_cast<hipStream_t>(stream));
 }
 
-extern "C" int attnlab_topk_tiled(const float* scores, int64_t score_stride, int R, int M, int k, int order,
-                                  int32_t* top_idx, float* top_val, int64_t top_stride, uint32_t* state, void* scratch,
-                                  int64_t scratch_bytes, void* stream) {
+int topk_tiled_impl(const float* scores, int64_t score_stride, int R, int M, int k, int order, int32_t* top_idx,
+                    int64_t* idx64, float* top_val, int64_t top_stride, uint32_t* state, void* scratch,
+                    int64_t scratch_bytes, void* stream) {
     ATTNLAB_REQUIRE(R >= 0 && M >= 0, "R=%d and M=%d must be non-negative", R, M);
     ATTNLAB_REQUIRE(0 <= k && k <= M, "need 0 <= k <= M, got k=%d M=%d", k, M);
     ATTNLAB_REQUIRE(order == ATTNLAB_ORDER_POSITION || order == ATTNLAB_ORDER_SCORE, "unknown order %d", order);
@@ -2019,7 +2053,7 @@ extern "C" int attnlab_topk_tiled(const float* scores, int64_t score_stride, int
     ATTNLAB_REQUIRE(scratch != nullptr && (reinterpret_cast<uintptr_t>(scratch) & 255) == 0 && scratch_bytes >= need,
                     "scratch must be 256-byte aligned and hold attnlab_select_scratch_bytes(%d, %d, %d, %d) = %lld bytes",
                     R, M, k, order, (long long)need);
-    SelectArgs a{scores, score_stride, M, k, 0, 0, 0, 1, 0, order, nullptr, 0, nullptr, top_idx, top_val, top_stride,
+    SelectArgs a{scores, score_stride, M, k, 0, 0, 0, 1, 0, order, nullptr, 0, idx64, top_idx, top_val, top_stride,
                  state};
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if ((M + 31) / 32 > kMaxWords) {   // rows past 262144 keys: single-workgroup select, which builds its own histograms
@@ -2027,6 +2061,32 @@ extern "C" int attnlab_topk_tiled(const float* scores, int64_t score_stride, int
         return run_select(a, R, false, scratch, s, false);
     }
     return run_select(a, R, true, scratch, s, true);
+}
+
+}  // namespace
+
+extern "C" int attnlab_topk(const float* scores, int64_t score_stride, int R, int M, int k, int order, int32_t* top_idx,
+                            float* top_val, int64_t top_stride, void* stream) {
+    return topk_impl(scores, score_stride, R, M, k, order, top_idx, nullptr, top_val, top_stride, stream);
+}
+
+extern "C" int attnlab_topk_tiled(const float* scores, int64_t score_stride, int R, int M, int k, int order,
+                                  int32_t* top_idx, float* top_val, int64_t top_stride, uint32_t* state, void* scratch,
+                                  int64_t scratch_bytes, void* stream) {
+    return topk_tiled_impl(scores, score_stride, R, M, k, order, top_idx, nullptr, top_val, top_stride, state, scratch,
+                           scratch_bytes, stream);
+}
+
+extern "C" int attnlab_topk_i64(const float* scores, int64_t score_stride, int R, int M, int k, int order,
+                                int64_t* top_idx, float* top_val, void* stream) {
+    return topk_impl(scores, score_stride, R, M, k, order, nullptr, top_idx, top_val, k, stream);
+}
+
+extern "C" int attnlab_topk_tiled_i64(const float* scores, int64_t score_stride, int R, int M, int k, int order,
+                                      int64_t* top_idx, float* top_val, uint32_t* state, void* scratch,
+                                      int64_t scratch_bytes, void* stream) {
+    return topk_tiled_impl(scores, score_stride, R, M, k, order, nullptr, top_idx, top_val, k, state, scratch,
+                           scratch_bytes, stream);
 }
 
 extern "C" int attnlab_select_rows(const float* scores, int64_t score_stride, int B, int G, int lo, int hi, int legal,

@@ -174,6 +174,12 @@ int attnlab_topk_tiled(const float* scores, int64_t score_stride, int R, int M, 
                        float* top_val, int64_t top_stride, uint32_t* state, void* scratch, int64_t scratch_bytes,
                        void* stream);
 
+/* The same two with int64 indices (torch.topk's index type); top_idx and top_val rows are k apart. */
+int attnlab_topk_i64(const float* scores, int64_t score_stride, int R, int M, int k, int order, int64_t* top_idx,
+                     float* top_val, void* stream);
+int attnlab_topk_tiled_i64(const float* scores, int64_t score_stride, int R, int M, int k, int order, int64_t* top_idx,
+                           float* top_val, uint32_t* state, void* scratch, int64_t scratch_bytes, void* stream);
+
 /*
  * Selection of one decode step: top-k over the candidate scores merged with the fixed set F, written as the row
  * list the attend kernel reads. Replaces select_rows_kernel + the optional canonical sort

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 import torch
 
+from attention_lab import _native as nat
 from attention_lab import hip_select
 from oracle import exact
 
@@ -324,3 +325,34 @@ def test_validation(gpu):
         hip_select.topk(t, 3, order="random")
     with pytest.raises(ValueError):
         hip_select.select_rows(torch.zeros(1, 8, 10, device=gpu), 4, 15, 20, 3, 32)   # M != hi - lo
+
+
+@pytest.mark.parametrize("M,k,tiled", [(1, 1, False), (1000, 31, False), (4097, 4097, False), (300000, 77, False),
+                                       (32769, 1025, True), (40001, 8192, True), (40001, 8193, True),
+                                       (262145, 9000, True)])
+@pytest.mark.parametrize("order", ["score", "position"])
+def test_int64_topk_is_the_int32_topk(gpu, M, k, tiled, order):
+    """attnlab_topk_i64 / attnlab_topk_tiled_i64 write the indices and values of the int32 entries (each sort of the
+    score order, the radix pass past its LDS, rows past the tiled limit), rows of odd length."""
+    if order == "score" and k > hip_select.LDS_SORT_K and not tiled:
+        pytest.skip("needs the tiled entry's scratch")
+    R = 3
+    s = torch.from_numpy(tie_heavy(np.random.default_rng(M + k), (R, M))).to(gpu)
+    code = hip_select.ORDERS[order]
+    i32 = torch.full((R, k + 1), -7, dtype=torch.int32, device=gpu)
+    v32 = torch.full((R, k + 1), -7.0, device=gpu)
+    args = [s.data_ptr(), M, R, M, k, code, i32.data_ptr(), v32.data_ptr(), k + 1]
+    stream = nat.stream_of(s.device)
+    if tiled:
+        state = torch.zeros(R, nat.SELECT_STATE_WORDS, dtype=torch.int32, device=gpu)
+        scratch = torch.empty(nat.lib().attnlab_select_scratch_bytes(R, M, k, code), dtype=torch.uint8, device=gpu)
+        nat.call("attnlab_topk_tiled", *args, state.data_ptr(), scratch.data_ptr(), scratch.numel(), stream)
+    else:
+        nat.call("attnlab_topk", *args, stream)
+    vals, idx = hip_select.topk(s, k, order=order, tiled=tiled)
+    torch.cuda.synchronize()
+    assert idx.dtype == torch.int64 and idx.is_contiguous()
+    assert torch.equal(i32[:, :k].long(), idx) and torch.equal(v32[:, :k], vals)
+    assert (i32[:, k] == -7).all() and (v32[:, k] == -7.0).all()
+    want = exact.topk(s.cpu().numpy(), k, order=order)
+    assert np.array_equal(idx.cpu().numpy(), want)
