@@ -15,13 +15,16 @@ inline int64_t align_up(int64_t x) { return (x + kAlign - 1) / kAlign * kAlign; 
 
 struct Layout {
     int64_t scores, rows, u, sel, part, total;
+    int64_t long_lists, full;   // the long rows' key lists, past what every other route needs; the size with them
     int64_t score_stride;
 };
 
 // Workspace layout: scores [BG, round_up(M, 4)] fp32 | rows [BG, S] int32 | u [BG, 32] fp32 | select scratch: either
 // the tiled select's bitmaps and candidate entries (and for k past the LDS sort the score-order sort's buffers, sized
 // for score order so either order fits) or the score kernel's per-workgroup key lists, whichever is larger, since a
-// step uses one of them | partials [BG, P, h, 130] fp32. Nothing here needs to start at zero. The select state
+// step uses one of them | partials [BG, P, h, 130] fp32 | the key lists of rows of 32769 to 131072 candidates, which the
+// step keeps beside the scores (a workspace without this last region takes the tiled select). Nothing here needs to
+// start at zero. The select state
 // (first-digit histograms, which must start at zero) lives in its own buffer: a region inside this shape-dependent
 // layout would overlap other data of a differently shaped earlier call.
 Layout layout_of(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
@@ -37,6 +40,13 @@ Layout layout_of(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
     const int64_t sel = k > 0 ? attnlab::select_scratch_bytes((int)BG, (int)M, k, ATTNLAB_ORDER_SCORE) : 0;
     L.part = L.sel + align_up(std::max(sel, attnlab::list_region_bytes(BG, lo, hi, k)));
     L.total = L.part + align_up(P > 1 ? BG * P * h * 130 * 4 : 0);
+    L.long_lists = L.total;
+    L.full = L.total;
+    if (M > attnlab::kListMaxM) {
+        const attnlab::FusedGeometry g = attnlab::fused_tiling((int)BG, lo, hi);
+        const attnlab::ListPlan p = attnlab::list_plan((int)M, k, g, attnlab::kListLongM);
+        if (p.cap > 0) L.full += align_up(attnlab::list_bytes((int)BG, g, p));
+    }
     return L;
 }
 
@@ -44,7 +54,7 @@ Layout layout_of(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
 
 extern "C" int64_t attnlab_sparse_decode_workspace(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
     if (B < 1 || G < 1 || h < 1 || lo < 0 || hi < lo || legal < hi || k < 0 || P < 1) return -1;
-    return layout_of(B, G, h, lo, hi, legal, k, P).total;
+    return layout_of(B, G, h, lo, hi, legal, k, P).full;
 }
 
 namespace {
@@ -99,20 +109,23 @@ int sparse_decode_step_impl(const uint16_t* q_main, const uint16_t* K, const uin
     if (k > 0 && state && hi - lo > kListMaxM && !rows_out && !rows_flat &&
         select_attend_applies(B, G, lo, hi, legal, k, h, P)) {
         // a longer row whose list stays in the call: the same two launches (score with lists, select and attend) instead
-        // of score, classify, resolve and attend. No score is stored then, and the lists take the scores' place (they
-        // fit there unless k is a large part of the row), so the workspace keeps its size. k = M / 32, per layer, four
-        // launches against two: 128K B=1 h=2 39.2 / 37.3 us, B=2 h=2 54.9 / 50.9, B=4 h=2 93.1 / 82.3; 64K B=1 h=2 28.7 /
-        // 26.4, B=4 h=4 52.1 / 48.5; 40K B=8 h=2 60.4 / 54.2.
+        // of score, classify, resolve and attend. k = M / 32, per layer, four launches against two: 128K B=1 h=2 39.2 / 37.3 us,
+        // B=2 h=2 54.9 / 51.3, B=4 h=2 93.1 / 82.3; 64K B=1 h=2 28.7 / 26.4, B=4 h=4 52.1 / 49.2; 40K B=8 h=2 60.4 / 54.2.
         const ListPlan lp = list_plan(hi - lo, k, geo, kListLongM);
-        if (lp.cap > 0 && list_bytes(B * G, geo, lp) <= L.rows - L.scores) {
+        if (lp.cap > 0 && list_bytes(B * G, geo, lp) <= workspace_bytes - L.long_lists) {
             plan = lp;
-            lists = list_layout(ws + L.scores, B * G, geo, lp);
+            lists = list_layout(ws + L.long_lists, B * G, geo, lp);
         }
     }
     // Stored scores are read only by the tiled select and by score order (which reads the picks' scores back to sort
     // them); the list select in position order recomputes the rare tile it needs from the table and u, so the score
-    // kernel then writes key lists only.
+    // kernel then writes key lists only. The
+    // keys of a tile whose list was cut go where the scores would (write_key_list).
     const bool store_scores = plan.cap == 0 || order == ATTNLAB_ORDER_SCORE;
+    if (!store_scores) {
+        lists.keys = reinterpret_cast<uint32_t*>(scores);
+        lists.key_stride = L.score_stride;
+    }
     float* u_ws = reinterpret_cast<float*>(ws + L.u);
     int rc;
     if (k > 0) {

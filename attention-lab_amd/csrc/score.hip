@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void score_scan_fused(ScoreArgs a) {
     }
     if (a.hist) flush_histogram<256>(hsh, a.hist, bg);
     if (a.lists.entries)
-        write_key_list<NSUB>(a.lists, hsh, lcount, lkey, lvalid, (size_t)bg * a.tiles + tile, cb0, sstride, lo);
+        write_key_list<NSUB>(a.lists, hsh, lcount, lkey, lvalid, bg, (size_t)bg * a.tiles + tile, cb0, sstride, lo);
 }
 
 // 2-byte-load scan for tables whose rows are not 16-byte aligned: thread -> 8 adjacent columns from lo, never

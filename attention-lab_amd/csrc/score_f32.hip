@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void score_scan_fused_f32(ScoreF32Args a) {
     }
     if (a.hist) flush_histogram<256>(hsh, a.hist, bg);
     if (a.lists.entries)
-        write_key_list<NSUB>(a.lists, hsh, lcount, lkey, lvalid, (size_t)bg * a.tiles + tile, cb0, sstride, lo);
+        write_key_list<NSUB>(a.lists, hsh, lcount, lkey, lvalid, bg, (size_t)bg * a.tiles + tile, cb0, sstride, lo);
 }
 
 // Bulk build: zT[bg, j, col0 + t] = wk[g, j, :] . k_pre[bg, t, :] in float32. Block = 4 waves over 64 positions;

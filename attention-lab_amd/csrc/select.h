@@ -72,7 +72,9 @@ __device__ __forceinline__ void clear_histogram(uint32_t* hsh) {
 // found by one wave on its own: lane l sums the l-th 32 bins from the top (starting at a lane-dependent 16-byte segment,
 // so the lanes spread over the LDS banks), a DPP scan finds the chunk, a second scan its bin. No barrier; every lane of
 // the calling wave gets the digit.
-__device__ __forceinline__ uint32_t wave_digit_of_rank(const uint32_t* hist, uint32_t rank) {
+// *at_least (where given): the keys of that digit and above.
+__device__ __forceinline__ uint32_t wave_digit_of_rank(const uint32_t* hist, uint32_t rank,
+                                                       uint32_t* at_least = nullptr) {
     const int lane = threadIdx.x & 63;
     const int top = kHistBins - 32 * (lane + 1);   // lane 0: the highest 32 bins
     uint32_t sum = 0;
@@ -83,6 +85,7 @@ __device__ __forceinline__ uint32_t wave_digit_of_rank(const uint32_t* hist, uin
     }
     const uint32_t inc = wave_incl_scan(sum);
     const uint64_t m = __ballot(inc >= rank);
+    if (at_least) *at_least = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
     if (m == 0) return 0u;
     const int l0 = __ffsll((unsigned long long)m) - 1;
     const uint32_t above = (uint32_t)__builtin_amdgcn_readlane((int)(inc - sum), l0);
@@ -90,7 +93,9 @@ __device__ __forceinline__ uint32_t wave_digit_of_rank(const uint32_t* hist, uin
     const uint32_t c = lane < 32 ? hist[hib - lane] : 0u;
     const uint32_t inc2 = wave_incl_scan(c) + above;
     const uint64_t m2 = __ballot(lane < 32 && inc2 >= rank);
-    return (uint32_t)(hib - (__ffsll((unsigned long long)m2) - 1));
+    const int l1 = __ffsll((unsigned long long)m2) - 1;
+    if (at_least) *at_least = (uint32_t)__builtin_amdgcn_readlane((int)inc2, l1);
+    return (uint32_t)(hib - l1);
 }
 
 // The index table a row's candidate scores come from, for the select of the fused step when the score kernel wrote
@@ -184,11 +189,13 @@ struct RowScores {
 // Per-workgroup key lists of the fused decode step (the score kernel writes them, the list select reads them): for
 // each score workgroup of a row, every key of its tile whose first digit is at least the digit of its lmin-th largest
 // key, as (candidate index, key) pairs, and a header (that digit, the list's length; a length above cap means the
-// list was cut and its tile must be read in full).
+// list was cut and its tile must be read in full: from `keys` where given, which holds every key of exactly those tiles).
 struct ScoreLists {
     uint2* entries;   // [B*G, tiles, cap]
     uint2* hdr;       // [B*G, tiles]
     int lmin, cap;
+    uint32_t* keys = nullptr;   // [B*G, key_stride], candidate m at [m]
+    int64_t key_stride = 0;
 };
 
 // The key list of one 256-thread score workgroup (list number `list`), called by every thread once the workgroup's
@@ -196,13 +203,16 @@ struct ScoreLists {
 // that of the tile's lmin-th largest key (each wave finds that digit itself, no barrier), in no particular order. A
 // wave reserves its entries with one LDS atomic on lcount[0]; the wave that finishes last (lcount[1]) writes the
 // header. Both counters start at zero. Thread t's keys: lkey[i] of column cb0 + (i / 2) * sstride + 2 t + i % 2, valid
-// where bit i of lvalid is set.
+// where bit i of lvalid is set. A tile with more keys than the list holds also stores all of them (L.keys): a row whose
+// keys crowd one first digit (scores with a common part, or all equal) is then selected from 4 bytes a candidate, not
+// recomputed at 64, and any other row stores nothing.
 template <int NSUB>
 __device__ __forceinline__ void write_key_list(const ScoreLists& L, const uint32_t* hsh, uint32_t* lcount,
-                                               const uint32_t (&lkey)[2 * NSUB], uint32_t lvalid, size_t list,
+                                               const uint32_t (&lkey)[2 * NSUB], uint32_t lvalid, int row, size_t list,
                                                int cb0, int sstride, int lo) {
     const int tid = threadIdx.x, lane = tid & 63;
-    const uint32_t dl = wave_digit_of_rank(hsh, (uint32_t)L.lmin);
+    uint32_t length;
+    const uint32_t dl = wave_digit_of_rank(hsh, (uint32_t)L.lmin, &length);
     uint32_t m = 0u;
 #pragma unroll
     for (int i = 0; i < 2 * NSUB; ++i) m |= (uint32_t)(((lvalid >> i) & 1u) && (lkey[i] >> kHistShift) >= dl) << i;
@@ -225,6 +235,12 @@ __device__ __forceinline__ void write_key_list(const ScoreLists& L, const uint32
     // after the fourth wave's "done"
     if (lane == 0 && __hip_atomic_fetch_add(&lcount[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 3)
         L.hdr[list] = make_uint2(dl, __hip_atomic_load(&lcount[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    if (L.keys && length > (uint32_t)L.cap) {
+        uint32_t* krow = L.keys + (size_t)row * L.key_stride;
+#pragma unroll
+        for (int i = 0; i < 2 * NSUB; ++i)
+            if ((lvalid >> i) & 1u) krow[cb0 + (i >> 1) * sstride + 2 * tid + (i & 1) - lo] = lkey[i];
+    }
 }
 
 // The argument checks of attnlab_select_rows (the decode step runs them before its first launch, so a rejected call

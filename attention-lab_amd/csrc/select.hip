@@ -1505,6 +1505,8 @@ struct ListArgs {
     const uint2* hdr;       // [R, tiles]
     int cap, tiles, nsub, lspl;
     TableRef table;         // where SelectArgs::scores is null: the table the scores are recomputed from
+    const uint32_t* keys;   // ... and the keys of the tiles whose list was cut (null: none stored)
+    int64_t key_stride;
 };
 
 template <int MAXSUB>
@@ -1540,6 +1542,7 @@ __global__ __launch_bounds__(kSelThreads) void select_lists(SelectArgs a, ListAr
     r.tiles = t.tiles;
     r.nsub = t.nsub;
     r.lspl = t.lspl;
+    r.keys = t.keys ? t.keys + (size_t)row * t.key_stride : nullptr;
     list_select_bitmap<kSelThreads, kListSlots, MAXSUB>(r, L);
     const uint32_t sw = L.bits[threadIdx.x];
     init_sortbuf(a, sh);   // score order: the staged pairs' padding (the candidates in sortbuf are no longer read)
@@ -1624,6 +1627,7 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     r.tiles = t.tiles;
     r.nsub = t.nsub;
     r.lspl = t.lspl;
+    r.keys = t.keys ? t.keys + (size_t)bg * t.key_stride : nullptr;
     list_select_bitmap<kSAThreads, SLOTS, MAXSUB, WORDS>(r, L);
     // this thread's selected candidates [64 kWPT tid, 64 kWPT (tid + 1)) and their first slot among the k picks
     uint64_t words[kWPT];
@@ -1927,7 +1931,7 @@ int select_lists_impl(const float* scores, int64_t score_stride, int B, int G, i
     SelectArgs a{scores, score_stride, M, k, lo, hi, legal, G, C, order, rows, rows_stride, rows_flat, nullptr, nullptr, 0,
                  state};
     ListArgs t{lists.entries, lists.hdr, lists.cap, geo.tiles, geo.nsub, list_lspl(geo.tiles, kSelWaves, kListSlots, lists.lmin),
-               recompute ? table : TableRef{}};
+               recompute ? table : TableRef{}, recompute ? lists.keys : nullptr, lists.key_stride};
     // the instance for up to four sub-tiles per score workgroup keeps fewer registers live
     if (geo.nsub <= 4) hipLaunchKernelGGL(select_lists<4>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
     else hipLaunchKernelGGL(select_lists<8>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
@@ -1964,7 +1968,8 @@ int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, ui
     SelectArgs sa{nullptr, 0, M, k, lo, hi, legal, G, C, ATTNLAB_ORDER_POSITION, nullptr, 0, nullptr, nullptr, nullptr, 0,
                   state};
     ListArgs t{lists.entries, lists.hdr, lists.cap, geo.tiles, geo.nsub,
-               list_lspl(geo.tiles, kSAWaves, M > kListMaxM ? kSALongSlots : kSASlots, lists.lmin), table};
+               list_lspl(geo.tiles, kSAWaves, M > kListMaxM ? kSALongSlots : kSASlots, lists.lmin), table, lists.keys,
+               lists.key_stride};
     const int Q = fused_head_groups(B * G, h, P);
     AttendArgs a{K, V, (int64_t)C * kHeadDim, kHeadDim, q, nullptr, 0, S, C, h, P, Q, scale * kLog2e, out, 1, part};
     if (P > 1) {

@@ -13,9 +13,9 @@
 //      (lo & ~7) + (s * tiles + w) * 512 + [0, 512));
 //   3. finds the second digit; when its bin holds exactly the keys still to take (the usual case) the selection is
 //      complete, else a third digit and the first krem tied keys in index order (a tie bitmap and one block scan).
-// A bin b1 holding more than kListCandCap keys is resolved by three radix passes over the row's scores instead. The
-// scores of an incomplete list's tile and of a radix-resolved row are the stored ones where the score stage wrote them,
-// else recomputed from the index table in the score kernel's exact operation order (rescore8). The result is the
+// A bin b1 holding more than kListCandCap keys is resolved by two or three radix passes over the row's keys instead. An
+// incomplete list's tile and a radix-resolved row are read from the scores or the keys the score stage stored, else
+// recomputed from the index table in the score kernel's exact operation order (rescore8). The result is the
 // selection bitmap in LDS (bit i: candidate i is among the top k; ties go to the lower index).
 #pragma once
 
@@ -38,6 +38,7 @@ struct ListRow {
     int M, k, lo, hi;
     int cap, tiles, nsub;
     int lspl;                 // log2 of the entries per lane and list loaded in the first round trip
+    const uint32_t* keys;     // the keys of tiles whose list was cut, where the scores are not stored (null: none)
 };
 
 // LDS of list_select_bitmap (the caller places the arrays, so that they can share memory with its other phases). Fill
@@ -166,45 +167,215 @@ __device__ __forceinline__ void take_ties(const ListLds& L, uint32_t krem) {
     __syncthreads();
 }
 
-// Bin b1 too full for the candidate array: the remaining two digits by passes over the row's scores, then every key
-// above the threshold and the first krem keys equal to it. Called by every thread with the same b1 and krem. The three
-// passes are one loop (pass 0: second digit of bin b1's keys; pass 1: third digit of prefix p2; pass 2: keys above
-// and equal to the threshold T into the two bitmaps), so the score read, possibly a recompute from the table, is
-// emitted once.
-template <int THREADS, int WORDS>
-__device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L, uint32_t b1, uint32_t krem) {
-    const int tid = threadIdx.x;
-    uint32_t prefix = b1;   // pass 0: the first digit; pass 1: the first two (p2); pass 2: the threshold key T
-#pragma unroll 1
-    for (int pass = 0; pass < 3; ++pass) {
-        for (int c0 = (r.lo & ~7) + 8 * tid; c0 < r.hi; c0 += 8 * THREADS) {
-            float v[8];
-            r.scores.group8(c0, v);
+// Bits [m0, m0 + 8) of a bitmap: mask's set bits join (m0 may start below 0, where mask is clear).
+__device__ __forceinline__ void or_bits8(uint32_t* bits, int m0, uint32_t mask) {
+    if (mask == 0u) return;
+    if (m0 < 0) {
+        mask >>= -m0;
+        m0 = 0;
+    }
+    const uint64_t w = (uint64_t)mask << (m0 & 31);
+    if ((uint32_t)w) atomicOr(&bits[m0 >> 5], (uint32_t)w);
+    if (w >> 32) atomicOr(&bits[(m0 >> 5) + 1], (uint32_t)(w >> 32));
+}
+
+// Pass 3's key of bin p2: counted, and appended to the candidates.
+__device__ __forceinline__ void radix_collect(const ListLds& L, uint32_t ix, uint32_t key) {
+    atomicAdd(&L.hist3[key & 1023u], 1u);
+    const uint32_t j = atomicAdd(&L.misc[0], 1u);
+    if (j < (uint32_t)kListCandCap) L.cand[j] = make_uint2(ix, key & 1023u);
+}
+
+// One radix pass over the keys of eight consecutive scores (candidates m0 .. m0 + 7, those with their ok bit set). pass 0: the second
+// digit of bin `prefix`'s keys; pass 1: the third digit of the keys with the first two digits `prefix`; pass 2: the keys
+// above and equal to `prefix` into the two bitmaps; pass 3 (in place of 1 and 2 where the keys with the first two digits
+// `prefix` fit the candidate array): the keys above those into the bitmap, those into the array, counted as in pass 1. A wave whose keys all
+// share one digit counts them with one atomic: the LDS adds of equal digits take turns, and a row of equal scores (an index not filled yet)
+// spends most of a pass in them otherwise.
+template <int PASS>
+__device__ __forceinline__ void radix_take8(const ListLds& L, uint32_t prefix, const uint32_t (&key)[8], uint32_t ok,
+                                            int m0) {
+    if constexpr (PASS == 3) {
+        uint32_t above = 0u;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int c = c0 + i;
-                if (c < r.lo || c >= r.hi) continue;
-                const uint32_t key = score_key(v[i]), m = (uint32_t)(c - r.lo);
-                if (pass == 0) {
-                    if ((key >> kHistShift) == prefix) atomicAdd(&L.hist2[(key >> 10) & 2047u], 1u);
-                } else if (pass == 1) {
-                    if ((key >> 10) == prefix) atomicAdd(&L.hist3[key & 1023u], 1u);
-                } else if (key > prefix) {   // both bitmaps start zeroed (the first round trip cleared them)
-                    atomicOr(&L.bits[m >> 5], 1u << (m & 31u));
-                } else if (key == prefix) {
-                    atomicOr(&L.ties[m >> 5], 1u << (m & 31u));
-                }
+        for (int i = 0; i < 8; ++i) above |= (uint32_t)((key[i] >> 10) > prefix) << i;
+        or_bits8(L.bits, m0, above & ok);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((key[i] >> 10) == prefix && ((ok >> i) & 1u)) radix_collect(L, (uint32_t)(m0 + i), key[i]);
+        return;
+    }
+    if constexpr (PASS == 2) {
+        uint32_t above = 0u, tie = 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            above |= (uint32_t)(key[i] > prefix) << i;
+            tie |= (uint32_t)(key[i] == prefix) << i;
+        }
+        or_bits8(L.bits, m0, above & ok);
+        or_bits8(L.ties, m0, tie & ok);
+        return;
+    }
+    uint32_t* h = PASS == 0 ? L.hist2 : L.hist3;
+    constexpr int top = PASS == 0 ? kHistShift : 10, down = PASS == 0 ? 10 : 0;
+    constexpr uint32_t dmask = PASS == 0 ? 2047u : 1023u;
+    bool same = ok == 0xffu && (key[0] >> top) == prefix;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) same = same && (key[i] >> down) == (key[0] >> down);
+    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(key[0] >> down));
+    const uint64_t active = __ballot(1);
+    if (__ballot(same && (key[0] >> down) == d0) == active) {
+        if ((int)(threadIdx.x & 63) == __ffsll((unsigned long long)active) - 1)
+            atomicAdd(&h[d0 & dmask], 8u * (uint32_t)__popcll(active));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if ((key[i] >> top) == prefix && ((ok >> i) & 1u)) atomicAdd(&h[(key[i] >> down) & dmask], 1u);
+}
+
+__device__ __forceinline__ void radix_take8(const ListLds& L, int pass, uint32_t prefix, const uint32_t (&key)[8],
+                                            uint32_t ok, int m0) {
+    if (pass == 0) radix_take8<0>(L, prefix, key, ok, m0);
+    else if (pass == 1) radix_take8<1>(L, prefix, key, ok, m0);
+    else if (pass == 2) radix_take8<2>(L, prefix, key, ok, m0);
+    else radix_take8<3>(L, prefix, key, ok, m0);
+}
+
+// Whether table columns [c0, c0 + 8) lie in a tile whose keys the score kernel stored (list w was cut), and those keys.
+__device__ __forceinline__ bool keys_stored(const ListRow& r, const ListLds& L, int w) {
+    return r.keys && L.hdr[w].y > (uint32_t)r.cap;
+}
+__device__ __forceinline__ void stored_keys8(const ListRow& r, int c0, uint32_t (&key)[8]) {
+    const uint32_t* p = r.keys + (c0 - r.lo);
+    if (c0 >= r.lo && c0 + 8 <= r.hi && (reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+        const uint4 x = *reinterpret_cast<const uint4*>(p), y = *reinterpret_cast<const uint4*>(p + 4);
+        key[0] = x.x; key[1] = x.y; key[2] = x.z; key[3] = x.w;
+        key[4] = y.x; key[5] = y.y; key[6] = y.z; key[7] = y.w;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) key[i] = c0 + i >= r.lo && c0 + i < r.hi ? p[i] : 0u;
+    }
+}
+
+// One radix pass over the stored keys: every 512-column block of a tile whose list was cut, kBlocks of a wave's in flight.
+template <int THREADS, int PASS>
+__device__ __forceinline__ void radix_stored(const ListRow& r, const ListLds& L, uint32_t prefix) {
+    constexpr int kWaves = THREADS / 64;
+    constexpr int kBlocks = 2;   // eight in flight were no faster
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lo8 = r.lo & ~7, nblk = (r.hi - lo8 + 511) / 512;
+#pragma unroll 1
+    for (int b0 = wave, w = wave; b0 < nblk; b0 += kBlocks * kWaves) {
+        uint32_t key[kBlocks][8], ok[kBlocks];
+#pragma unroll
+        for (int u = 0; u < kBlocks; ++u) {
+            const int blk = b0 + kWaves * u, c0 = lo8 + 512 * blk + 8 * lane;
+            while (w >= r.tiles) w -= r.tiles;   // the block's list
+            const bool stored = blk < nblk && keys_stored(r, L, w);
+            w += kWaves;
+            ok[u] = 0u;
+            if (stored) {
+                stored_keys8(r, c0, key[u]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) ok[u] |= (uint32_t)(c0 + i >= r.lo && c0 + i < r.hi) << i;
             }
         }
+#pragma unroll
+        for (int u = 0; u < kBlocks; ++u) {
+            const int m0 = lo8 + 512 * (b0 + kWaves * u) + 8 * lane - r.lo;
+            if (ok[u]) radix_take8<PASS>(L, prefix, key[u], ok[u], m0);
+        }
+    }
+}
+
+// Bin b1 too full for the candidate array: the remaining two digits by passes over the row's keys (two, or three where the
+// second digit leaves more than the candidate array holds), then every key above
+// the threshold and the first krem keys equal to it. Called by every thread with the same b1 and krem. A wave takes 512
+// table columns at a time, which lie in one tile: where the tile's list was cut, from its stored keys, several blocks
+// in flight (reading 4 stored bytes a candidate against recomputing it from 64 in every workgroup of the row: index rows
+// with a common part, B=8 h=4 at 32K 175 -> 68 us a step, B=2 h=2 at 128K 397 -> 106; equal rows 150 -> 73, 430 -> 129;
+// rows that crowd no digit pay 0.1-0.2 us for the longer kernels); where it is complete down to b1, from the list; else from the scores, stored or recomputed.
+template <int THREADS, int WORDS>
+__device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L, uint32_t b1, uint32_t krem) {
+    constexpr int kWaves = THREADS / 64;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lo8 = r.lo & ~7;
+    uint32_t prefix = b1;   // pass 0: the first digit; pass 1: the first two (p2); pass 2: the threshold key T
+    bool other = r.scores.srow || !r.keys;   // some tile is read from its list or its scores
+    for (int w = lane; w < r.tiles; w += 64) other = other || !keys_stored(r, L, w);
+    const int nother = __any(other) ? r.nsub * r.tiles : 0;   // also blocks past hi: a list's entries are shared by its blocks
+    int pass = 0;
+#pragma unroll 1
+    while (true) {
+#pragma unroll 1
+        for (int blk = wave, sub = 0, w = wave; blk < nother; blk += kWaves, w += kWaves) {
+            for (; w >= r.tiles; w -= r.tiles) ++sub;   // block 512 blk: sub-tile sub of list w
+            const int c0 = lo8 + 512 * blk + 8 * lane;
+            if (!r.scores.srow) {
+                if (keys_stored(r, L, w)) continue;
+                const uint2 h = L.hdr[w];
+                if (h.x <= b1 && h.y <= (uint32_t)r.cap) {
+                    const uint2* ep = r.entries + (size_t)w * r.cap;
+                    for (int j = 64 * sub + lane; j < (int)h.y; j += 64 * r.nsub) {
+                        const uint2 e = ep[j];
+                        const uint32_t ix = min(e.x, (uint32_t)r.M - 1u), key = e.y;   // in range for any list contents
+                        if (pass == 0) {
+                            if ((key >> kHistShift) == prefix) atomicAdd(&L.hist2[(key >> 10) & 2047u], 1u);
+                        } else if (pass == 1) {
+                            if ((key >> 10) == prefix) atomicAdd(&L.hist3[key & 1023u], 1u);
+                        } else if (pass == 3) {
+                            if ((key >> 10) == prefix) radix_collect(L, ix, key);
+                            else if ((key >> 10) > prefix) atomicOr(&L.bits[ix >> 5], 1u << (ix & 31u));
+                        } else if (key > prefix) {
+                            atomicOr(&L.bits[ix >> 5], 1u << (ix & 31u));
+                        } else if (key == prefix) {
+                            atomicOr(&L.ties[ix >> 5], 1u << (ix & 31u));
+                        }
+                    }
+                    continue;
+                }
+            }
+            if (c0 >= r.hi) continue;
+            float v[8];
+            r.scores.group8(c0, v);
+            uint32_t key[8], ok = 0u;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                key[i] = score_key(v[i]);
+                ok |= (uint32_t)(c0 + i >= r.lo && c0 + i < r.hi) << i;
+            }
+            radix_take8(L, pass, prefix, key, ok, c0 - r.lo);
+        }
+        if (!r.scores.srow && r.keys) {
+            if (pass == 0) radix_stored<THREADS, 0>(r, L, prefix);
+            else if (pass == 1) radix_stored<THREADS, 1>(r, L, prefix);
+            else if (pass == 2) radix_stored<THREADS, 2>(r, L, prefix);
+            else radix_stored<THREADS, 3>(r, L, prefix);
+        }
         __syncthreads();
+        if (pass == 2) break;
         if (pass == 0) {
             wave0_find_digit(L.misc + 1, L.hist2, krem, 2048);
             prefix = (b1 << 11) | (L.misc[1] & 2047u);
-        } else if (pass == 1) {
-            wave0_find_digit(L.misc + 1, L.hist3, krem, 1024);
-            prefix = (prefix << 10) | (L.misc[1] & 1023u);
+            krem = L.misc[2];
+            pass = L.misc[3] <= (uint32_t)kListCandCap ? 3 : 1;   // keys of bin p2
+            continue;   // misc is written next after the pass's barrier
         }
-        krem = pass < 2 ? L.misc[2] : krem;
+        wave0_find_digit(L.misc + 1, L.hist3, krem, 1024);
+        const uint32_t d3 = L.misc[1] & 1023u;
+        krem = L.misc[2];
+        if (pass == 3) {
+            const uint32_t nc = min(L.misc[0], (uint32_t)kListCandCap);
+            for (uint32_t j = threadIdx.x; j < nc; j += THREADS) {
+                const uint2 c = L.cand[j];
+                if (c.y >= d3) atomicOr(&(c.y > d3 ? L.bits : L.ties)[c.x >> 5], 1u << (c.x & 31u));
+            }
+            __syncthreads();
+            break;
+        }
+        prefix = (prefix << 10) | d3;
+        pass = 2;
     }
     take_ties<THREADS, WORDS>(L, krem);
 }
@@ -373,8 +544,9 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
         const int items = nf * r.nsub * 64;
         for (int q0 = 64 * wave; q0 < items; q0 += 64 * kWaves) {
             const int q = q0 + lane;
-            float v[8];
+            uint32_t key[8];
             int c0 = 0;
+            bool stored = false;
             if (q < items) {
                 int nth = q / (64 * r.nsub);   // the nth incomplete list (its number: the nth set bit of f0, f1)
                 uint64_t m = f0;
@@ -388,18 +560,25 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
                 const int wl = base + __ffsll((unsigned long long)m) - 1;
                 const int sb = (q / 64) % r.nsub;
                 c0 = (r.lo & ~7) + (sb * nt + wl) * 512 + (q % 64) * 8;
+                stored = keys_stored(r, L, wl);
             }
-            if (q < items && c0 < r.hi) {
-                r.scores.group8(c0, v);
+            if (q < items && c0 < r.hi && stored) {
+                stored_keys8(r, c0, key);
             } else {
+                float v[8];
+                if (q < items && c0 < r.hi) {
+                    r.scores.group8(c0, v);
+                } else {
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+                    for (int i = 0; i < 8; ++i) v[i] = 0.0f;
+                }
+#pragma unroll
+                for (int i = 0; i < 8; ++i) key[i] = score_key(v[i]);
             }
-            uint32_t idx[8], key[8], ok = 0u;
+            uint32_t idx[8], ok = 0u;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int c = c0 + i;
-                key[i] = score_key(v[i]);
                 idx[i] = (uint32_t)(c - r.lo);
                 ok |= (uint32_t)(q < items && c >= r.lo && c < r.hi) << i;
             }

@@ -689,3 +689,51 @@ def test_fused_select_attend_on_rows_past_32768(gpu, B, G, h, L, rho, case, P):
     separate attend, bit for bit, and the float64 oracle; the score distributions that leave lists incomplete or crowd
     the threshold's bin take the recomputed tiles and the radix passes."""
     test_fused_select_attend_equals_the_separate_stages(gpu, B, G, h, -(-L // 8) * 8, L, rho, case, P)
+
+
+@pytest.mark.parametrize("B,G,h,L,rho,dtype", [
+    (1, 2, 2, 131072 + 68, 1 / 32, torch.bfloat16),   # every tile's keys stored
+    (1, 2, 2, 40003, 1 / 32, torch.bfloat16),         # ragged: the last block partly past the row
+    (2, 2, 4, 70000, 1 / 32, torch.float32),
+    (1, 8, 2, 32768, 1 / 32, torch.bfloat16),
+    (1, 3, 2, 30001, 1 / 8, torch.float32),
+])
+@pytest.mark.parametrize("kind", ["common", "third", "equal"])
+def test_rows_that_crowd_one_first_digit(gpu, B, G, h, L, rho, dtype, kind):
+    """More than 8192 keys share the threshold's first digit: index rows with a common part (two radix passes), such
+    rows in a random third of the 512-column blocks (their tiles' keys stored or listed, the others' lists complete) and
+    equal rows (three passes, ties by index). The fused step equals the step that returns its rows, bit for bit (past
+    32768 candidates the tiled select, which reads stored scores), and those rows equal the oracle's."""
+    from attention_lab import _native as nat
+    C = -(-L // 8) * 8
+    ws = nat.Workspace()
+    K, V, q, q_pre, k_pre_new, zT, idx = setup(gpu, B=B, G=G, h=h, C=C, seed=L + h)
+    req = prepare_request(B, G, C, valid_length=L, query_position=L - 1, rho=rho, device=gpu)
+    lo, hi = req.layout.candidate_lo, req.layout.candidate_hi
+    # a common part along u, so that every score moves by about four of its standard deviations
+    u = torch.einsum("bgd,gdr->bgr", q_pre.float().reshape(B, G, -1).cpu(), idx.wq_t_scaled.float().cpu()).to(gpu)
+    part = (4.0 * u / u.norm(dim=-1, keepdim=True))[..., None]
+    z = zT.float()
+    if kind == "common":
+        z = z + part
+    elif kind == "third":
+        blocks = torch.rand(-(-C // 512), generator=torch.Generator().manual_seed(L)) < 1 / 3
+        z = z + part * blocks.repeat_interleave(512)[:C].to(gpu)
+    else:
+        z[..., lo:hi] = z[..., lo:lo + 1]
+    zT = z.to(dtype)
+    wq, wk, qp, kn = (t.to(dtype) for t in (idx.wq_t_scaled, idx.wk, q_pre, k_pre_new))
+    outs = []
+    for rows in (False, True):
+        got = sparse_decode_step_kernel(q, qp, K, V, zT.clone(), wq, wk, req.fixed_rows, req.off_lo, lo, hi, req.k,
+                                        req.selected_count, k_pre_new=kn, write_col=req.write_col, return_rows=rows,
+                                        canonical_order=True, workspace=ws)
+        torch.cuda.synchronize()
+        assert int(ws.bytes(gpu, 0, "state").abs().sum()) == 0, f"rows={rows}: the select state left dirty"
+        outs.append(got[0] if rows else got)
+    assert torch.equal(outs[0], outs[1])
+    pos = (got[1].view(B, G, req.selected_count) - req.offsets).cpu().numpy()
+    if kind == "equal":
+        want = np.concatenate([np.arange(lo + req.k), np.arange(hi, L)])
+        assert (pos == want).all()
+    check_out(outs[0], exact.subset_attention(f64(q)[:, :, :, 0], f64(K), f64(V), pos), f"{kind} L={L}")
