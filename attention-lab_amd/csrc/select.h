@@ -166,15 +166,16 @@ __device__ __forceinline__ void rescore8(const TableRef& t, int bg, int c0, floa
 }
 
 // A row's candidate scores for the select: read from the stored scores where the score stage wrote them (srow,
-// candidate index m at srow[m]), else recomputed from the index table. group8 gives table columns c0 .. c0 + 7
-// (c0 % 8 == 0); entries outside [lo, hi) are 0 and must be masked by the caller.
+// candidate index m at srow[m]), else (srow null) recomputed from the index table. group8 gives table columns c0 .. c0 + 7
+// (c0 % 8 == 0); entries outside [lo, hi) are 0 and must be masked by the caller. SCORES: whether srow is given.
 struct RowScores {
     const float* srow;
     TableRef table;
     int bg, lo, hi;
 
+    template <bool SCORES>
     __device__ __forceinline__ void group8(int c0, float (&s)[8]) const {
-        if (srow) {
+        if constexpr (SCORES) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const int c = c0 + i;
@@ -235,7 +236,7 @@ __device__ __forceinline__ void write_key_list(const ScoreLists& L, const uint32
     // after the fourth wave's "done"
     if (lane == 0 && __hip_atomic_fetch_add(&lcount[1], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP) == 3)
         L.hdr[list] = make_uint2(dl, __hip_atomic_load(&lcount[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
-    if (L.keys && length > (uint32_t)L.cap) {
+    if (__builtin_expect(length > (uint32_t)L.cap && L.keys, 0)) {
         uint32_t* krow = L.keys + (size_t)row * L.key_stride;
 #pragma unroll
         for (int i = 0; i < 2 * NSUB; ++i)

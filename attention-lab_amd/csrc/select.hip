@@ -1518,6 +1518,9 @@ __global__ __launch_bounds__(kSelThreads) void select_lists(SelectArgs a, ListAr
     __shared__ uint32_t misc[4];
     static_assert(kListCandCap * sizeof(uint2) <= sizeof(SelectShared::sortbuf), "candidates live in sortbuf");
     const int row = xcd_contiguous_block();   // the XCD whose score workgroups wrote the row
+    a.top_idx = nullptr;   // a row list only; without stored scores in position order (select_lists_impl checks it): an
+    a.top_val = nullptr;   // instance holds no code for the rest
+    if constexpr (MAXSUB == 0) a.order = ATTNLAB_ORDER_POSITION;
     ListLds L;
     L.hist = sh.hist;
     L.hist2 = lds;
@@ -1576,7 +1579,7 @@ constexpr int kSAStages = 3;
 constexpr int kSAReadCounter = kSelectStateWords - 1;   // the row's readers of its bins: the last arrival word
 static_assert(kListWords == 2 * kSAThreads, "two selection bitmap words per thread");
 
-template <int MAXSUB, int H, int WORDS = kListWords, int SLOTS = kSASlots>
+template <int H, int WORDS = kListWords, int SLOTS = kSASlots>
 __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListArgs t, AttendArgs a) {
     constexpr int kWPT = WORDS / (2 * kSAThreads);   // 64-bit bitmap words per thread
     __shared__ __attribute__((aligned(16))) uint32_t hist[kHistBins];
@@ -1615,7 +1618,7 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     L.misc = misc;
     L.wave_tot = wave_tot;
     ListRow r;
-    r.scores = RowScores{sa.scores ? sa.scores + (size_t)bg * sa.score_stride : nullptr, t.table, bg, sa.lo, sa.hi};
+    r.scores = RowScores{nullptr, t.table, bg, sa.lo, sa.hi};   // such a step stores no scores
     r.state = sa.hist + (size_t)bg * kSelectStateWords;
     r.entries = t.entries + (size_t)bg * t.tiles * t.cap;
     r.hdr = t.hdr + (size_t)bg * t.tiles;
@@ -1628,7 +1631,7 @@ __global__ __launch_bounds__(kSAThreads) void select_attend(SelectArgs sa, ListA
     r.nsub = t.nsub;
     r.lspl = t.lspl;
     r.keys = t.keys ? t.keys + (size_t)bg * t.key_stride : nullptr;
-    list_select_bitmap<kSAThreads, SLOTS, MAXSUB, WORDS>(r, L);
+    list_select_bitmap<kSAThreads, SLOTS, 0, WORDS>(r, L);
     // this thread's selected candidates [64 kWPT tid, 64 kWPT (tid + 1)) and their first slot among the k picks
     uint64_t words[kWPT];
     uint32_t x = 0u;
@@ -1932,8 +1935,9 @@ int select_lists_impl(const float* scores, int64_t score_stride, int B, int G, i
                  state};
     ListArgs t{lists.entries, lists.hdr, lists.cap, geo.tiles, geo.nsub, list_lspl(geo.tiles, kSelWaves, kListSlots, lists.lmin),
                recompute ? table : TableRef{}, recompute ? lists.keys : nullptr, lists.key_stride};
-    // the instance for up to four sub-tiles per score workgroup keeps fewer registers live
-    if (geo.nsub <= 4) hipLaunchKernelGGL(select_lists<4>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
+    // without stored scores, or with them: for up to four sub-tiles per score workgroup fewer registers are live
+    if (recompute) hipLaunchKernelGGL(select_lists<0>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
+    else if (geo.nsub <= 4) hipLaunchKernelGGL(select_lists<4>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
     else hipLaunchKernelGGL(select_lists<8>, dim3(B * G), dim3(kSelThreads), 0, stream, a, t);
     return check_launch("select_lists");
 }
@@ -1978,18 +1982,16 @@ int select_attend_impl(int B, int G, int lo, int hi, int legal, int k, int C, ui
     }
     const dim3 grid(B * G * Q * P), block(kSAThreads);
     const int hq = h / Q;
-#define SA_LAUNCH(MS)                                                                                     \
-    do {                                                                                                  \
-        if (hq == 1) hipLaunchKernelGGL((select_attend<MS, 1>), grid, block, 0, stream, sa, t, a);        \
-        else if (hq == 2) hipLaunchKernelGGL((select_attend<MS, 2>), grid, block, 0, stream, sa, t, a);   \
-        else hipLaunchKernelGGL((select_attend<MS, 4>), grid, block, 0, stream, sa, t, a);                \
-    } while (0)
+#define SA_LAUNCH(...) hipLaunchKernelGGL((select_attend<__VA_ARGS__>), grid, block, 0, stream, sa, t, a)
     if (M > kListMaxM) {
-        if (hq == 1) hipLaunchKernelGGL((select_attend<8, 1, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
-        else if (hq == 2) hipLaunchKernelGGL((select_attend<8, 2, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
-        else hipLaunchKernelGGL((select_attend<8, 4, kListLongWords, kSALongSlots>), grid, block, 0, stream, sa, t, a);
-    } else if (geo.nsub <= 4) SA_LAUNCH(4);
-    else SA_LAUNCH(8);
+        if (hq == 1) SA_LAUNCH(1, kListLongWords, kSALongSlots);
+        else if (hq == 2) SA_LAUNCH(2, kListLongWords, kSALongSlots);
+        else SA_LAUNCH(4, kListLongWords, kSALongSlots);
+    } else {
+        if (hq == 1) SA_LAUNCH(1);
+        else if (hq == 2) SA_LAUNCH(2);
+        else SA_LAUNCH(4);
+    }
 #undef SA_LAUNCH
     return check_launch("select_attend");
 }

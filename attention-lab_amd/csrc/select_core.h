@@ -186,12 +186,12 @@ __device__ __forceinline__ void radix_collect(const ListLds& L, uint32_t ix, uin
     if (j < (uint32_t)kListCandCap) L.cand[j] = make_uint2(ix, key & 1023u);
 }
 
-// One radix pass over the keys of eight consecutive scores (candidates m0 .. m0 + 7, those with their ok bit set). pass 0: the second
-// digit of bin `prefix`'s keys; pass 1: the third digit of the keys with the first two digits `prefix`; pass 2: the keys
-// above and equal to `prefix` into the two bitmaps; pass 3 (in place of 1 and 2 where the keys with the first two digits
-// `prefix` fit the candidate array): the keys above those into the bitmap, those into the array, counted as in pass 1. A wave whose keys all
-// share one digit counts them with one atomic: the LDS adds of equal digits take turns, and a row of equal scores (an index not filled yet)
-// spends most of a pass in them otherwise.
+// One radix pass over the keys of eight consecutive scores (candidates m0 .. m0 + 7, those with their ok bit set). pass 0:
+// the second digit of bin `prefix`'s keys; pass 1: the third digit of the keys with the first two digits `prefix`; pass 2:
+// the keys above and equal to `prefix` into the two bitmaps; pass 3 (in place of 1 and 2 where the keys with the first two
+// digits `prefix` fit the candidate array): the keys above those into the bitmap, those into the array, counted as in pass
+// 1. A wave whose keys all share one digit counts them with one atomic: the LDS adds of equal digits take turns, and a row
+// of equal scores (an index not filled yet) spends most of a pass in them otherwise.
 template <int PASS>
 __device__ __forceinline__ void radix_take8(const ListLds& L, uint32_t prefix, const uint32_t (&key)[8], uint32_t ok,
                                             int m0) {
@@ -234,12 +234,46 @@ __device__ __forceinline__ void radix_take8(const ListLds& L, uint32_t prefix, c
         if ((key[i] >> top) == prefix && ((ok >> i) & 1u)) atomicAdd(&h[(key[i] >> down) & dmask], 1u);
 }
 
+// The same with the pass as a value: for the blocks that are not read from stored keys, whose lists or recomputed scores
+// bound the pass (an instance per pass there as well was 5 KB of code in every kernel, and no faster).
 __device__ __forceinline__ void radix_take8(const ListLds& L, int pass, uint32_t prefix, const uint32_t (&key)[8],
                                             uint32_t ok, int m0) {
-    if (pass == 0) radix_take8<0>(L, prefix, key, ok, m0);
-    else if (pass == 1) radix_take8<1>(L, prefix, key, ok, m0);
-    else if (pass == 2) radix_take8<2>(L, prefix, key, ok, m0);
-    else radix_take8<3>(L, prefix, key, ok, m0);
+    if (pass >= 2) {
+        const int sh = pass == 3 ? 10 : 0;
+        uint32_t above = 0u, equal = 0u;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            above |= (uint32_t)((key[i] >> sh) > prefix) << i;
+            equal |= (uint32_t)((key[i] >> sh) == prefix) << i;
+        }
+        or_bits8(L.bits, m0, above & ok);
+        equal &= ok;
+        if (pass == 2) {
+            or_bits8(L.ties, m0, equal);
+            return;
+        }
+        if (equal == 0u) return;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if ((equal >> i) & 1u) radix_collect(L, (uint32_t)(m0 + i), key[i]);
+        return;
+    }
+    uint32_t* h = pass == 0 ? L.hist2 : L.hist3;
+    const int top = pass == 0 ? kHistShift : 10, down = pass == 0 ? 10 : 0;
+    const uint32_t dmask = pass == 0 ? 2047u : 1023u;
+    bool same = ok == 0xffu && (key[0] >> top) == prefix;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) same = same && (key[i] >> down) == (key[0] >> down);
+    const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)(key[0] >> down));
+    const uint64_t active = __ballot(1);
+    if (__ballot(same && (key[0] >> down) == d0) == active) {
+        if ((int)(threadIdx.x & 63) == __ffsll((unsigned long long)active) - 1)
+            atomicAdd(&h[d0 & dmask], 8u * (uint32_t)__popcll(active));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if ((key[i] >> top) == prefix && ((ok >> i) & 1u)) atomicAdd(&h[(key[i] >> down) & dmask], 1u);
 }
 
 // Whether table columns [c0, c0 + 8) lie in a tile whose keys the score kernel stored (list w was cut), and those keys.
@@ -290,19 +324,20 @@ __device__ __forceinline__ void radix_stored(const ListRow& r, const ListLds& L,
 }
 
 // Bin b1 too full for the candidate array: the remaining two digits by passes over the row's keys (two, or three where the
-// second digit leaves more than the candidate array holds), then every key above
-// the threshold and the first krem keys equal to it. Called by every thread with the same b1 and krem. A wave takes 512
-// table columns at a time, which lie in one tile: where the tile's list was cut, from its stored keys, several blocks
-// in flight (reading 4 stored bytes a candidate against recomputing it from 64 in every workgroup of the row: index rows
-// with a common part, B=8 h=4 at 32K 175 -> 68 us a step, B=2 h=2 at 128K 397 -> 106; equal rows 150 -> 73, 430 -> 129;
-// rows that crowd no digit pay 0.1-0.2 us for the longer kernels); where it is complete down to b1, from the list; else from the scores, stored or recomputed.
-template <int THREADS, int WORDS>
+// second digit leaves more than the candidate array holds), then every key above the threshold and the first krem keys
+// equal to it. Called by every thread with the same b1 and krem. A wave takes 512 table columns at a time, which lie in one
+// tile. SCORES: from the stored scores. Else, where the tile's list was cut, from its stored keys, several blocks in flight;
+// where it is complete down to b1, from the list; else recomputed. Reading 4 stored bytes a candidate against recomputing
+// it from 64 in every workgroup of the row, per layer: index rows with a common part, B=8 h=4 at 32K 190.8 -> 63.7 us, B=2
+// h=2 at 128K 556 -> 119; equal rows 153 -> 69 and 428 -> 125. Rows that crowd no digit pay nothing at 32K (B=1 18.9 both)
+// and up to 0.5 us past 32768 candidates (B=1 64K 26.0 -> 26.5).
+template <int THREADS, int WORDS, bool SCORES>
 __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L, uint32_t b1, uint32_t krem) {
     constexpr int kWaves = THREADS / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lo8 = r.lo & ~7;
     uint32_t prefix = b1;   // pass 0: the first digit; pass 1: the first two (p2); pass 2: the threshold key T
-    bool other = r.scores.srow || !r.keys;   // some tile is read from its list or its scores
+    bool other = SCORES || !r.keys;   // some tile is read from its list or its scores
     for (int w = lane; w < r.tiles; w += 64) other = other || !keys_stored(r, L, w);
     const int nother = __any(other) ? r.nsub * r.tiles : 0;   // also blocks past hi: a list's entries are shared by its blocks
     int pass = 0;
@@ -312,7 +347,7 @@ __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L,
         for (int blk = wave, sub = 0, w = wave; blk < nother; blk += kWaves, w += kWaves) {
             for (; w >= r.tiles; w -= r.tiles) ++sub;   // block 512 blk: sub-tile sub of list w
             const int c0 = lo8 + 512 * blk + 8 * lane;
-            if (!r.scores.srow) {
+            if constexpr (!SCORES) {
                 if (keys_stored(r, L, w)) continue;
                 const uint2 h = L.hdr[w];
                 if (h.x <= b1 && h.y <= (uint32_t)r.cap) {
@@ -338,7 +373,7 @@ __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L,
             }
             if (c0 >= r.hi) continue;
             float v[8];
-            r.scores.group8(c0, v);
+            r.scores.group8<SCORES>(c0, v);
             uint32_t key[8], ok = 0u;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -347,11 +382,13 @@ __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L,
             }
             radix_take8(L, pass, prefix, key, ok, c0 - r.lo);
         }
-        if (!r.scores.srow && r.keys) {
-            if (pass == 0) radix_stored<THREADS, 0>(r, L, prefix);
-            else if (pass == 1) radix_stored<THREADS, 1>(r, L, prefix);
-            else if (pass == 2) radix_stored<THREADS, 2>(r, L, prefix);
-            else radix_stored<THREADS, 3>(r, L, prefix);
+        if constexpr (!SCORES) {
+            if (r.keys) {
+                if (pass == 0) radix_stored<THREADS, 0>(r, L, prefix);
+                else if (pass == 1) radix_stored<THREADS, 1>(r, L, prefix);
+                else if (pass == 2) radix_stored<THREADS, 2>(r, L, prefix);
+                else radix_stored<THREADS, 3>(r, L, prefix);
+            }
         }
         __syncthreads();
         if (pass == 2) break;
@@ -383,10 +420,15 @@ __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L,
 // The selection bitmap of one row (in L.bits, complete and synchronised on return). SLOTS: entries per lane loaded
 // in the first round trip (the first 64 << r.lspl entries of each of the wave's first SLOTS >> r.lspl lists; later
 // entries and lists are read afterwards). MAXSUB (4 or 8): the most sub-tiles per score workgroup this instance reads
-// for an incomplete list (r.nsub <= MAXSUB). Called by every thread of the workgroup.
+// from the stored scores of an incomplete list (r.nsub <= MAXSUB; r.scores.srow is given); 0: the scores are not stored
+// (srow is null; any r.nsub). An instance holds the code of one of the two only, since the length of the code costs every
+// step: with both in one kernel the one-head select and attend was 70 KB (56 now) and a layer at 32K, B=1 took 0.15 to 0.25
+// us more (28 layers 538.6 / 531.4 us; B=5, 12K, float32 187.9 / 185.8; B=2, 128K, 4 layers 206.0 / 203.8; a step that
+// returns its rows, B=1, 21.2 / 20.7). Called by every thread of the workgroup.
 template <int THREADS, int SLOTS, int MAXSUB, int WORDS = kListWords>
 __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListLds& L) {
-    static_assert(MAXSUB == 4 || MAXSUB == 8, "sub-tiles are read four at a time");
+    static_assert(MAXSUB == 0 || MAXSUB == 4 || MAXSUB == 8, "sub-tiles are read four at a time");
+    constexpr bool kScores = MAXSUB > 0;
     constexpr int kWaves = THREADS / 64;
     constexpr int W = WORDS / THREADS;
     static_assert(SLOTS % 8 == 0, "slots are taken in passes of 8");
@@ -430,8 +472,8 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
     uint32_t above, nb1;
     const uint32_t b1 = wave_first_digit(sbv, L.hist, (uint32_t)r.k, above, nb1);
     uint32_t krem = (uint32_t)r.k - above;
-    if (nb1 > (uint32_t)kListCandCap) {   // the same test in every wave
-        radix_bitmap<THREADS, WORDS>(r, L, b1, krem);
+    if (__builtin_expect(nb1 > (uint32_t)kListCandCap, 0)) {   // the same test in every wave
+        radix_bitmap<THREADS, WORDS, kScores>(r, L, b1, krem);
         return;
     }
     const uint32_t M = (uint32_t)r.M;
@@ -498,9 +540,7 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
                 }
                 take(idx, key, ok, 8);
             }
-        } else if (!r.scores.srow) {
-            // an incomplete list whose scores were not stored: its tile is recomputed by every thread below
-        } else {
+        } else if constexpr (kScores) {   // (without stored scores: by every thread below)
             // an incomplete list: the tile's stored scores, lane -> 8 consecutive columns of each sub-tile, four
             // sub-tiles' loads issued before the first is used
             const float* srow = r.scores.srow;
@@ -532,8 +572,8 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
             }
         }
     }
-    if (!r.scores.srow) {
-        // The tiles of the incomplete lists, recomputed from the index table by the whole workgroup: a wave takes 64
+    if constexpr (!kScores) {
+        // The tiles of the incomplete lists, from their stored keys or recomputed, by the whole workgroup: a wave takes 64
         // groups of 8 columns at a time (group q: list = the (q / (64 nsub))-th incomplete one, sub-tile
         // (q / 64) % nsub, columns 8 (q % 64) .. + 8 of it). Every wave reads the same headers, so the lists agree.
         const uint2 h0 = lane < nt ? L.hdr[lane] : make_uint2(0u, 0u);
@@ -567,7 +607,7 @@ __device__ __forceinline__ void list_select_bitmap(const ListRow& r, const ListL
             } else {
                 float v[8];
                 if (q < items && c0 < r.hi) {
-                    r.scores.group8(c0, v);
+                    rescore8(r.scores.table, r.scores.bg, c0, v);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 8; ++i) v[i] = 0.0f;
