@@ -50,10 +50,14 @@ Layout layout_of(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
     return L;
 }
 
+bool step_sizes_ok(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
+    return B >= 1 && G >= 1 && h >= 1 && lo >= 0 && hi >= lo && legal >= hi && k >= 0 && P >= 1;
+}
+
 }  // namespace
 
 extern "C" int64_t attnlab_sparse_decode_workspace(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
-    if (B < 1 || G < 1 || h < 1 || lo < 0 || hi < lo || legal < hi || k < 0 || P < 1) return -1;
+    if (!step_sizes_ok(B, G, h, lo, hi, legal, k, P)) return -1;
     return layout_of(B, G, h, lo, hi, legal, k, P).full;
 }
 
@@ -235,7 +239,8 @@ extern "C" int attnlab_sparse_decode_step_noalloc(const uint16_t* q_main, const 
     using namespace attnlab;
     ATTNLAB_REQUIRE(B >= 1 && G >= 1 && (int64_t)B * G <= kNoAllocRows, "B*G=%lld rows exceed the %d of the no-allocation "
                     "entry point", (long long)B * G, kNoAllocRows);
-    const int64_t ws = attnlab_sparse_decode_workspace(B, G, h, lo, hi, legal, k, P);
+    // what the step cannot do without: long rows whose key lists don't fit beside it take the tiled select
+    const int64_t ws = step_sizes_ok(B, G, h, lo, hi, legal, k, P) ? layout_of(B, G, h, lo, hi, legal, k, P).total : -1;
     ATTNLAB_REQUIRE(ws >= 0, "invalid sizes B=%d G=%d h=%d lo=%d hi=%d legal=%d k=%d P=%d", B, G, h, lo, hi, legal, k, P);
     ATTNLAB_REQUIRE(kNoAllocStateBytes + ws <= kNoAllocBytes, "this step needs %lld bytes of workspace; the no-allocation "
                     "entry point holds %lld", (long long)ws, (long long)(kNoAllocBytes - kNoAllocStateBytes));

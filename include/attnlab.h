@@ -303,7 +303,9 @@ int attnlab_prefill_attend_split(const uint16_t* q, const uint16_t* K, const uin
 
 /*
  * Workspace (bytes) of attnlab_sparse_decode_step for these sizes: candidate scores, row list, u, tiled-select
- * scratch and split-K partials, each 256-byte aligned. Its contents need no initialisation.
+ * scratch and split-K partials, each 256-byte aligned, then the key lists of rows of 32769 to 131072 candidates. Its
+ * contents need no initialisation. A step of such rows also takes a workspace without that last region (and then selects
+ * tiled, with the same result); a workspace smaller than the rest is refused.
  */
 int64_t attnlab_sparse_decode_workspace(int B, int G, int h, int lo, int hi, int legal, int k, int P);
 
@@ -350,8 +352,8 @@ int attnlab_sparse_decode_step_f32(const uint16_t* q_main, const float* q_cat, c
  * the reference: it is for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc). The select state and the workspace live in a 32 MiB file-scope device array
  * that each device holds until the process ends; its first 256 * ATTNLAB_SELECT_STATE_WORDS words are the select state
- * (B*G <= 256), the rest the workspace (attnlab_sparse_decode_workspace of these sizes must fit, or the call returns
- * ATTNLAB_EINVAL). Arguments and outputs as in attnlab_sparse_decode_step (bf16 index table). Every call on a device
+ * (B*G <= 256), the rest the workspace (attnlab_sparse_decode_workspace of these sizes, or that without the long rows'
+ * key lists, must fit, or the call returns ATTNLAB_EINVAL). Arguments and outputs as in attnlab_sparse_decode_step (bf16 index table). Every call on a device
  * shares that device's array: calls that overlap on one device race, so order them on one stream.
  */
 int attnlab_sparse_decode_step_noalloc(const uint16_t* q_main, const uint16_t* q_cat, const uint16_t* K,

@@ -159,3 +159,22 @@ def test_list_select_refuses_shapes_it_does_not_cover(native_lib):
         _native.call("attnlab_select_lists", None, 2000, 1, 8, 4, 2004, 2068, 64, 2104, 0, 16, 200, None, 16, 256,
                      1 << 20, None, 0, 16, None)
     assert native_lib.attnlab_sparse_decode_workspace(0, 8, 2, 4, 100, 164, 3, 1) == -1
+
+
+@pytest.mark.parametrize("B,L", [(6, 131072), (8, 98304), (9, 98304), (12, 65536), (13, 65536), (21, 40960)])
+def test_no_alloc_step_takes_what_fits_without_the_long_rows_lists(native_lib, B, L):
+    """The no-allocation step's 32 MiB hold these steps but not the key lists of their long rows, which the step does
+    without (the tiled select): the size check lets them pass, so that here, without a device, the call ends at
+    hipGetDevice. One request more at 128K is past the step's own need."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the arguments are not device pointers: for a host without a device")
+    lo, hi, k = 4, L - 64, L // 32
+    held = (32 << 20) - 256 * _native.SELECT_STATE_WORDS * 4
+    args = lambda b: [*([16] * 8), b, 8, 2, 32, L, lo, hi, L, k, L - 1, 0.1, 0, 1, None, None, 16, None]  # noqa: E731
+    assert native_lib.attnlab_sparse_decode_workspace(B, 8, 2, lo, hi, L, k, 1) > held
+    with pytest.raises(RuntimeError, match="hipGetDevice"):
+        _native.call("attnlab_sparse_decode_step_noalloc", *args(B))
+    if L == 131072:
+        with pytest.raises(ValueError, match="no-allocation"):
+            _native.call("attnlab_sparse_decode_step_noalloc", *args(B + 1))

@@ -81,6 +81,25 @@ def test_no_alloc_step_without_rows_matches_the_step(gpu):
             assert torch.equal(a, b), f"call {n + 1}: {name} differs from attnlab_sparse_decode_step"
 
 
+def test_no_alloc_step_of_long_rows_without_room_for_their_lists(gpu):
+    """Six requests of 128K: the library's array holds the step but not the key lists of its rows, so this call takes the
+    tiled select and the separate attend where the step with a workspace of its own selects and attends in one launch. The
+    same output bits, and a smaller call afterwards (its state left zero)."""
+    B, h, C, L = 6, 2, 131072, 131072
+    gen = torch.Generator(device=gpu).manual_seed(77)
+    t = lambda *s: torch.randn(*s, generator=gen, device=gpu, dtype=torch.bfloat16)  # noqa: E731
+    idx = GroupedIndexer(8, h, 128, 32, device=gpu, dtype=torch.bfloat16, seed=77)
+    x = dict(q=t(B, 8, h, 128), q_cat=t(B, 8, h * 128), K=t(B, 8, C, 128), V=t(B, 8, C, 128), zT=t(B, 8, 32, C),
+             k_new=t(B, 8, 128), wq_t=idx.wq_t_scaled.contiguous(), wk=idx.wk.contiguous())
+    want = step(gpu, x, B, h, C, L, 1 / 32, nat.ORDER_POSITION, noalloc=False, with_rows=False)
+    got = step(gpu, x, B, h, C, L, 1 / 32, nat.ORDER_POSITION, noalloc=True, with_rows=False)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[3], want[3])
+    x = inputs(gpu, 1, 2, 2048 + 64, seed=78)
+    want = step(gpu, x, 1, 2, 2048 + 64, 2048, 1 / 16, nat.ORDER_SCORE, noalloc=False)
+    got = step(gpu, x, 1, 2, 2048 + 64, 2048, 1 / 16, nat.ORDER_SCORE, noalloc=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_no_alloc_refuses_more_than_it_holds(gpu):
     B, h, C, L = 40, 2, 64, 64        # 320 rows of select state: more than its 256
     x = inputs(gpu, 1, 1, 64, seed=1)
