@@ -23,7 +23,8 @@ struct Layout {
 // the tiled select's bitmaps and candidate entries (and for k past the LDS sort the score-order sort's buffers, sized
 // for score order so either order fits) or the score kernel's per-workgroup key lists, whichever is larger, since a
 // step uses one of them | partials [BG, P, h, 130] fp32 | the key lists of rows of 32769 to 131072 candidates, which the
-// step keeps beside the scores (a workspace without this last region takes the tiled select). Nothing here needs to
+// step keeps beside the scores where it can select and attend in one launch (a workspace without this last region takes the
+// tiled select). Nothing here needs to
 // start at zero. The select state
 // (first-digit histograms, which must start at zero) lives in its own buffer: a region inside this shape-dependent
 // layout would overlap other data of a differently shaped earlier call.
@@ -42,7 +43,9 @@ Layout layout_of(int B, int G, int h, int lo, int hi, int legal, int k, int P) {
     L.total = L.part + align_up(P > 1 ? BG * P * h * 130 * 4 : 0);
     L.long_lists = L.total;
     L.full = L.total;
-    if (M > attnlab::kListMaxM) {
+    // only where the step can run the select and attend that reads them
+    if (M > attnlab::kListMaxM && (int64_t)h * 128 <= attnlab::kFusedMaxHd &&
+        attnlab::select_attend_applies(B, G, lo, hi, legal, k, h, P)) {
         const attnlab::FusedGeometry g = attnlab::fused_tiling((int)BG, lo, hi);
         const attnlab::ListPlan p = attnlab::list_plan((int)M, k, g, attnlab::kListLongM);
         if (p.cap > 0) L.full += align_up(attnlab::list_bytes((int)BG, g, p));

@@ -810,7 +810,7 @@ extern "C" int attnlab_score_grouped(uint16_t* zT, const uint16_t* k_new, const 
 
 FusedGeometry attnlab::fused_geometry(int BG, int C, int r, int hd, int lo, int hi, const void* zT, bool u_given) {
     const bool v16_table = (C % 8 == 0) && (reinterpret_cast<uintptr_t>(zT) % 16 == 0);
-    if (u_given || !v16_table || r != 32 || hd > 512 || hi <= lo) return FusedGeometry{0, 0};
+    if (u_given || !v16_table || r != 32 || hd > kFusedMaxHd || hi <= lo) return FusedGeometry{0, 0};
     return fused_tiling(BG, lo, hi);
 }
 

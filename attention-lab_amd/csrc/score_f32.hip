@@ -482,7 +482,7 @@ __global__ __launch_bounds__(256) void project_keys_f32_mfma(ProjectF32Args a) {
 FusedGeometry fused_geometry_f32(int BG, int C, int r, int hd, int lo, int hi, const void* zT, const void* wq_t,
                                  bool u_given) {
     const bool table = C % 8 == 0 && reinterpret_cast<uintptr_t>(zT) % 16 == 0;
-    const bool u_ok = u_given || (hd >= 1 && hd <= 512 && reinterpret_cast<uintptr_t>(wq_t) % 16 == 0);
+    const bool u_ok = u_given || (hd >= 1 && hd <= kFusedMaxHd && reinterpret_cast<uintptr_t>(wq_t) % 16 == 0);
     if (!table || !u_ok || r != 32 || hi <= lo) return FusedGeometry{0, 0};
     return fused_tiling(BG, lo, hi);
 }

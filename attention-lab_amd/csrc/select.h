@@ -268,7 +268,9 @@ int score_grouped_impl(uint16_t* zT, const uint16_t* k_new, const uint16_t* wk, 
                        hipStream_t stream, const ScoreLists* lists = nullptr);
 
 // The one-launch score's tiling of a row (u, z column and scan in one kernel): sub-tiles of 512 columns per workgroup
-// and workgroups per row; nsub == 0 when that kernel does not apply (u given, unaligned table, r != 32, h*d > 512).
+// and workgroups per row; nsub == 0 when that kernel does not apply (u given, unaligned table, r != 32, h*d past
+// kFusedMaxHd).
+constexpr int kFusedMaxHd = 512;
 struct FusedGeometry {
     int nsub, tiles;
 };

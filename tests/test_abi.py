@@ -10,6 +10,7 @@ from pathlib import Path
 import pytest
 
 from attention_lab import _native
+from plans import list_bytes, list_cap, one_launch
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "attnlab.h"
 
@@ -178,3 +179,26 @@ def test_no_alloc_step_takes_what_fits_without_the_long_rows_lists(native_lib, B
     if L == 131072:
         with pytest.raises(ValueError, match="no-allocation"):
             _native.call("attnlab_sparse_decode_step_noalloc", *args(B + 1))
+
+
+@pytest.mark.parametrize("B,G,h,L,k,P,lists", [
+    (1, 8, 2, 131072, 4096, 16, True), (2, 8, 4, 131072 + 68, 4096, 8, True), (6, 8, 2, 131072, 4096, 5, True),
+    (1, 8, 1, 40003, 1250, 8, True), (4, 8, 4, 65536, 2048, 4, True), (1, 1, 2, 40000, 1200, 1, True),
+    (2, 8, 3, 131072, 4096, 8, False),       # three heads per workgroup: not a select and attend in one launch
+    (2, 8, 8, 131072, 4096, 8, False),       # eight heads: not the one-launch score, which writes the lists
+    (1, 8, 2, 131072, 8400, 1, False),       # 8468 rows of one partition: past what its LDS holds
+    (1, 8, 2, 131072, 8400, 2, True),
+    (1, 1, 2, 131000, 4096, 16, False),      # 256 score workgroups per row
+    (1, 8, 2, 131072 + 69, 4096, 16, False), # one candidate past the longest such row
+    (1, 8, 2, 131072, 66000, 16, False),     # lists of more than half a tile
+])
+def test_workspace_holds_long_rows_lists_where_a_step_can_read_them(native_lib, B, G, h, L, k, P, lists):
+    """Rows past 32768 candidates: the workspace's last region, and the rule of tests/plans.py for the shapes with one."""
+    lo, hi, BG = 4, L - 64, B * G
+    M, S = hi - lo, 68 + k
+    base = _a(BG * ((M + 3) // 4 * 4) * 4) + _a(BG * S * 4) + _a(BG * 32 * 4) + _a(select_scratch(BG, M, k, 1))
+    base += _a(BG * P * h * 130 * 4) if P > 1 else 0
+    assert one_launch(BG, lo, hi, L, k, h, P) == lists
+    assert native_lib.attnlab_sparse_decode_workspace(B, G, h, lo, hi, L, k, P) == \
+        base + (list_bytes(BG, lo, hi, k) if lists else 0)
+    assert list_cap(BG, lo, hi, k, 32768) == 0
