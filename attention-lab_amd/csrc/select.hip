@@ -137,13 +137,14 @@ __device__ __forceinline__ int sort_len(int k) {
     return n;
 }
 
-// Score order: fill sortbuf[0, sort_len(k)) with 0, below every staged (key, ~index) pair (~index > 0 for any
-// index < 2^32 - 1), so the padding sorts last. Ordered before the emission by the barriers of the block scan that
+// Score order: fill sortbuf[0, sort_len(k)) with 0, 1, 2, ..., below every staged (key, ~index) pair (~index is larger for
+// any row), so the padding sorts last, and no two pairs are equal, which bin_sort_desc's ranks rely on (a state that does
+// not match the scores leaves padding among the k). Ordered before the emission by the barriers of the block scan that
 // follows.
 __device__ __forceinline__ void init_sortbuf(const SelectArgs& a, SelectShared& sh) {
     if (a.order != ATTNLAB_ORDER_SCORE) return;
     const int n = sort_len(a.k);
-    for (int i = threadIdx.x; i < n; i += kSelThreads) sh.sortbuf[i] = 0ull;
+    for (int i = threadIdx.x; i < n; i += kSelThreads) sh.sortbuf[i] = (uint64_t)i;
 }
 
 // Bitonic sort of buf[0, n), descending, n a power of two >= 128. Every compare-exchange whose partner lies in the same
@@ -297,9 +298,8 @@ __device__ __forceinline__ const uint64_t* radix_sort_desc_1024(SelectShared& sh
 // Score order for k <= 1024 E staged pairs in slots [0, k), when the keys spread out: one pass into 4096 bins that are
 // linear in the key over [kmin, kmax] (bin = (kmax - key) >> s, with s the smallest shift that leaves at most 4096 bins,
 // so bin order is descending key order), then each pair's rank inside its bin by comparison with the bin's other pairs,
-// larger (key, ~index) first (pairs are distinct: their indices are; only slots that a histogram which does not match
-// the scores left at zero could be equal, and those may then repeat or miss a pair). The top k of a smooth score distribution puts a few
-// pairs in a bin; when a bin holds more than kBinSortMax (ties, outliers that stretch the key range), nothing has been
+// larger (key, ~index) first (pairs are distinct: their indices are, and init_sortbuf's padding is). The top k of a smooth
+// score distribution puts a few pairs in a bin; when a bin holds more than kBinSortMax (ties, outliers that stretch the key range), nothing has been
 // moved yet and the function returns false for the caller's other sort. The pairs wait in registers (E per thread)
 // between the phases, so they are sorted in place; the bins are 16-bit counters, two per word of sh.hist, turned into
 // each bin's first slot and then counted up to its end, which is the next bin's first slot.
@@ -546,7 +546,8 @@ __device__ __forceinline__ void finish_row(const SelectArgs& a, int row, SelectS
         float* tv = a.top_val + (size_t)row * a.top_stride;
         for (int j = tid; j < k; j += kSelThreads) {
             const uint64_t e = sh.sortbuf[j];
-            const int idx = min((int)(uint32_t)e, a.M - 1);   // in range for any slot left unwritten
+            // clamped as in score order: a slot left unwritten holds whatever the memory held
+            const int idx = min(max((int)(uint32_t)e, 0), a.M - 1);
             if (ti) ti[j] = idx;
             tv[j] = __uint_as_float((uint32_t)(e >> 32));
             if (flat) flat[lo + j] = base + lo + idx;

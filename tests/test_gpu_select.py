@@ -356,3 +356,36 @@ def test_int64_topk_is_the_int32_topk(gpu, M, k, tiled, order):
     assert (i32[:, k] == -7).all() and (v32[:, k] == -7.0).all()
     want = exact.topk(s.cpu().numpy(), k, order=order)
     assert np.array_equal(idx.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("order", ["position", "score"])
+@pytest.mark.parametrize("M,k", [(5000, 300), (5000, 3000), (40000, 1000)])
+def test_a_state_that_does_not_match_the_scores_gives_positions_of_the_row(gpu, M, k, order):
+    """A select state that counts keys the rows don't have leaves output slots unwritten: each still names a position of
+    its row (the picks that are written, once each), and the state ends zero. A score-order top-k before it leaves pairs in
+    the workgroups' memory whose low words are no positions."""
+    R = 512
+    g = torch.Generator(device=gpu).manual_seed(M + k)
+    # exponents spread, so that score order's bins don't crowd
+    s = torch.exp2(torch.rand(R, M, generator=g, device=gpu) * 60 - 30)
+    hip_select.topk(s, k, order="score", tiled=True)
+    over = k // 3
+    state = torch.zeros(R, nat.SELECT_STATE_WORDS, dtype=torch.int32, device=gpu)
+    state[:, 2047] = over        # keys of the highest first digit, which no score has
+    state[:, 2048 + 63] = over   # and their super-bin
+    code = hip_select.ORDERS[order]
+    idx = torch.full((R, k), -7, dtype=torch.int64, device=gpu)
+    val = torch.empty(R, k, device=gpu)
+    scratch = torch.empty(nat.lib().attnlab_select_scratch_bytes(R, M, k, code), dtype=torch.uint8, device=gpu)
+    nat.call("attnlab_topk_tiled_i64", s.data_ptr(), M, R, M, k, code, idx.data_ptr(), val.data_ptr(), state.data_ptr(),
+             scratch.data_ptr(), scratch.numel(), nat.stream_of(s.device))
+    torch.cuda.synchronize()
+    assert int(state.abs().sum()) == 0
+    assert int(idx.min()) >= 0 and int(idx.max()) < M
+    # the picks that were written are the row's largest
+    want = s.topk(k // 3, dim=1).values
+    got = s.gather(1, idx) if order == "score" else s.gather(1, idx).sort(dim=1, descending=True).values
+    if order == "score":
+        assert torch.equal(got[:, :k // 3], want)
+    for r in (0, R - 1):
+        assert torch.isin(want[r], got[r]).all()
