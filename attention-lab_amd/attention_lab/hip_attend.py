@@ -195,7 +195,7 @@ def sparse_partitions(BG: int, rows: int, h: int = 1, merged: bool = False) -> i
     return auto_partitions(BG * hg, rows, max_p=MAX_P, min_rows=128, blocks=blocks)
 
 
-def merged_partitions(BG: int, rows: int, h: int = 1) -> int:
+def merged_partitions(BG: int, rows: int, h: int = 1, one_launch: bool = True) -> int:
     """Split-K count of the fused step's attend (partials merged in-kernel by the last partition to arrive): one round
     of at most 256 workgroups (a workgroup of the one-launch select and attend fills a CU), split by rows first and by
     head groups after (the kernel adds head groups, which read the same rows again, while the grid stays within 256;
@@ -207,10 +207,32 @@ def merged_partitions(BG: int, rows: int, h: int = 1) -> int:
     against the grids of up to two rounds it replaces: 32K (S = 1092) B=3 h=2 26.6 against 34.1 us, B=5 h=4 38.6 /
     46.9, B=7 h=2 40.2 / 48.4, B=12 h=1 55.6 / 63.9; 12K (S = 454) B=5 h=4 22.3 / 30.3, B=12 h=2 37.0 / 44.1, B=24
     h=1 51.4 / 60.4; 3K (S = 162) B=12 h=4 20.6 / 26.7, B=2 h=4 14.5 at P=1 against 15.7 at P=2; B = 1, 2, 16 at 32K
-    as before. The largest miss against the best of all these: 0.8 us (32K, B=12, h=4)."""
+    as before. The largest miss against the best of all these: 0.8 us (32K, B=12, h=4).
+    Between 200 and 448 rows (h = 1, 2, 4, B = 1..5), P=1 is best at S = 224 (15.0 us, any split costs 0.2-1.5), and at
+    S = 271, 324, 380 and 443 this rule's P = 2 or 3 is 0.3-1.0 us slower than P = 4 to 8 at B <= 2 (S = 324, B=1 h=2:
+    16.2 against 15.4).
+    one_launch = False: a step that selects and attends in launches of their own (one_launch_step), whose attend
+    workgroups are small and several to a CU. With four heads per KV group the smaller grid loses there: 256 workgroups
+    or more, two head groups first from 32 (b, g) rows on (rows returned, S = 1092: B=12 65.9 against 72.1 us, B=7 47.3
+    / 49.3; S = 4164, B=3 79.1 / 85.6; S = 5068, 94.4 / 103.1). With eight, partitions of at least 256 rows (37 shapes
+    of 4K to 160K, B = 1..24, mean loss against the best P 0.9 %, where 128 rows lose 2.1 in either grid; S = 324, B=8
+    34.0 against 37.5). With other h the rule above is the better one there too: h=1 0.8 % where the larger grid loses
+    1.8, h=2 1.5 / 1.8, h=3 1.1 / 3.1, h=6 3.7 / 8.8."""
     hg = h & -h if h > 0 else 1
+    if hg == 4 and not one_launch:
+        return auto_partitions(BG * (2 if BG >= 32 else 1), rows, max_p=8, min_rows=128, blocks=256)
+    if hg == 8 and not one_launch:
+        return max(1, min(8, rows // 256, 256 // (max(BG, 1) * 2)))
     by_rows = rows // 128 if rows < 448 else max(8, rows // 128)
     return max(1, min(8 if hg >= 4 else 16, by_rows, 256 // (max(BG, 1) * (2 if hg >= 4 else 1))))
+
+
+def one_launch_step(h: int, candidates: int, rows_returned: bool) -> bool:
+    """Whether a step of these sizes can select and attend in one launch (decode.hip), which the split-K rule depends on:
+    its row list stays in the call, one, two or four heads per KV group (h * 128 <= 512 is also the one-launch score's
+    limit), at most 131072 candidates. A step that misses a further condition there (an unaligned table, k past about
+    0.4 of the candidates, more than 128 score workgroups per row) takes this rule's P too."""
+    return not rows_returned and h in (1, 2, 4) and candidates <= 131072
 
 
 def dense_partitions(BG: int, length: int) -> int:

@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import pytest
 
-from attention_lab.hip_attend import merged_partitions, sparse_partitions
+from attention_lab.hip_attend import merged_partitions, one_launch_step, sparse_partitions
 
 
 @pytest.mark.parametrize("BG,S,h,want", [
@@ -36,3 +36,22 @@ def test_merged_rule_never_asks_for_a_second_round(h):
             P = merged_partitions(BG, S, h)
             assert 1 <= P <= max(1, min(16, S // 56))
             assert P == 1 or BG * P <= 256
+
+
+@pytest.mark.parametrize("BG,S,h,want", [
+    (24, 1092, 4, 8), (40, 1092, 4, 4), (56, 1092, 4, 3), (96, 1092, 4, 2), (24, 4164, 4, 8), (24, 5068, 4, 8),
+    (96, 454, 4, 2), (8, 324, 8, 1), (24, 1092, 8, 4), (16, 454, 8, 1),
+])
+def test_steps_of_separate_launches_keep_the_grid_their_attend_was_measured_with(BG, S, h, want):
+    """A step whose rows are returned, or past what one launch selects and attends: at four heads per KV group the attend's
+    small workgroups want more partitions than one round of the one-launch kernel's, at eight longer ones; other h as
+    there."""
+    assert merged_partitions(BG, S, h, one_launch=False) == want != merged_partitions(BG, S, h)
+    for other in (1, 2, 3, 5, 6, 7):
+        assert merged_partitions(BG, S, other, one_launch=False) == merged_partitions(BG, S, other)
+
+
+def test_which_steps_run_in_one_launch():
+    assert one_launch_step(4, 32700, False) and one_launch_step(1, 131072, False)
+    assert not one_launch_step(4, 32700, True) and not one_launch_step(4, 131073, False)
+    assert not any(one_launch_step(h, 32700, False) for h in (3, 5, 6, 7, 8))
