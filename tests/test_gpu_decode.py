@@ -8,10 +8,13 @@ the dense read, legal <= 68 degenerates to the dense read, rows are original pos
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import pytest
 import torch
 
+import plans
 from attention_lab import hip_attend, hip_score, hip_select
 from attention_lab.decode import (dense_decode_step, gathered_decode_step_kernel, prepare_request,
                                   select_rows_kernel, sparse_decode_step, sparse_decode_step_kernel)
@@ -673,66 +676,145 @@ def test_fused_select_attend_equals_the_separate_stages(gpu, B, G, h, C, L, rho,
     check_out(outs[0], exact.subset_attention(f64(q)[:, :, :, 0], f64(K), f64(V), want), f"{case} P={P}")
 
 
-@pytest.mark.parametrize("B,G,h,L,rho,case,P", [
-    (1, 2, 2, 32768 + 69, 1 / 32, None, None),          # one candidate past the shorter instance's bitmap
-    (1, 8, 1, 40003, 1 / 32, None, None),
-    (2, 3, 4, 131072 + 68, 1 / 32, None, None),         # the longest row: every word of its bitmap
-    (1, 2, 2, 131072 + 69, 1 / 32, None, None),         # one past it: the separate launches on both sides
-    (1, 2, 8, 65536, 1 / 64, None, 3),                  # odd partitions, four heads per workgroup
-    (1, 1, 2, 131000, 1 / 16, None, 1),                 # one partition of 8254 rows: not taken
-    (1, 2, 2, 100001, 1 / 32, "all_equal", None),
-    (1, 2, 2, 100001, 1 / 32, "skewed_tile", 2),
-    (2, 2, 1, 70000, 1 / 32, "seven_values", None),
+@pytest.mark.parametrize("B,G,h,L,rho,case,P,fused", [
+    (1, 2, 2, 32768 + 69, 1 / 32, None, None, True),     # one candidate past the shorter instance's bitmap
+    (1, 8, 1, 40003, 1 / 32, None, None, True),
+    (1, 8, 2, 131072 + 68, 1 / 32, None, None, True),    # the longest row: every word of its bitmap, eight sub-tiles
+    (2, 3, 4, 131072 + 68, 1 / 32, None, None, True),    # ... and four per score workgroup
+    (1, 2, 2, 131072 + 69, 1 / 32, None, None, False),   # one past it: the separate launches on both sides
+    (2, 8, 4, 65536, 1 / 64, None, 9, True),             # odd partitions, four heads per workgroup
+    (1, 8, 2, 131000, 1 / 16, None, 1, False),           # one partition of 8255 rows: not taken
+    (1, 8, 2, 131000, 1 / 16, None, 2, True),
+    (1, 8, 2, 100001, 1 / 32, "all_equal", None, True),
+    (1, 8, 2, 131072, 1 / 32, "skewed_tile", 2, True),
+    (2, 2, 1, 70000, 1 / 32, "seven_values", None, True),
 ])
-def test_fused_select_attend_on_rows_past_32768(gpu, B, G, h, L, rho, case, P):
-    """The longer rows' instance (a 4096-word bitmap, the lists in the scores' place) against the tiled select and the
-    separate attend, bit for bit, and the float64 oracle; the score distributions that leave lists incomplete or crowd
-    the threshold's bin take the recomputed tiles and the radix passes."""
+def test_fused_select_attend_on_rows_past_32768(gpu, B, G, h, L, rho, case, P, fused):
+    """The longer rows' instance (a 4096-word bitmap, the lists in a region of the workspace of their own) against the tiled
+    select and the separate attend, bit for bit, and the float64 oracle. `fused`: whether the shape reaches it."""
+    req = prepare_request(B, G, -(-L // 8) * 8, valid_length=L, query_position=L - 1, rho=rho, device=gpu)
+    lo, hi = req.layout.candidate_lo, req.layout.candidate_hi
+    if P is None:   # one count for both sides: the partitions set the order of the sums
+        P = hip_attend.merged_partitions(B * G, req.selected_count, h)
+    assert plans.one_launch(B * G, lo, hi, L, req.k, h, P) == fused
     test_fused_select_attend_equals_the_separate_stages(gpu, B, G, h, -(-L // 8) * 8, L, rho, case, P)
 
 
+@pytest.mark.parametrize("B,G,h,L,dtype", [
+    (1, 8, 2, 131072, torch.bfloat16),        # eight sub-tiles per score workgroup
+    (1, 4, 4, 131072 + 68, torch.bfloat16),   # four, the longest row
+    (1, 8, 2, 70000, torch.float32),
+    (1, 2, 1, 40003, torch.bfloat16),         # one
+])
+@pytest.mark.parametrize("kind", ["recomputed", "stored", "both"])
+def test_long_rows_with_incomplete_lists(gpu, B, G, h, L, dtype, kind):
+    """Rows past 32768 candidates with tiles whose list misses part of the selection: a 512-column block far above the rest
+    (the list's last digit lies above the threshold's: the tile is recomputed from the table) and a block of equal largest
+    columns (the list is cut: the tile's stored keys are read, ties included). Rows and output against the oracle on the
+    score kernel's scores and, bit for bit, against the separate launches; plans.list_paths shows that the tiles are read
+    the way the case names."""
+    from attention_lab import _native as nat
+    C = -(-L // 8) * 8
+    gen = torch.Generator(device=gpu).manual_seed(L + h)
+    t = lambda *s: torch.randn(*s, generator=gen, device=gpu).to(torch.bfloat16)  # noqa: E731
+    K, V, q, q_pre, k_new, zT = t(B, G, C, 128), t(B, G, C, 128), t(B, G, h, 1, 128), t(B, G, h, 1, 128), t(B, G, 1, 128), \
+        t(B, G, 32, C)
+    idx = GroupedIndexer(G, h, 128, 32, device=gpu, dtype=torch.bfloat16, seed=L)
+    req = prepare_request(B, G, C, valid_length=L, query_position=L - 1, rho=1 / 32, device=gpu)
+    lo, hi, k, S = req.layout.candidate_lo, req.layout.candidate_hi, req.k, req.selected_count
+    zT, q_pre, k_new, wq, wk = (x.to(dtype) for x in (zT, q_pre, k_new, idx.wq_t_scaled, idx.wk))
+    if kind != "stored":
+        zT[..., 512 * 5:512 * 6] *= 64
+    if kind != "recomputed":
+        u = torch.einsum("bgf,gfr->bgr", q_pre.double().reshape(B, G, -1), wq.double())
+        best = torch.einsum("bgr,bgrm->bgm", u, zT[..., lo:hi].double()).argmax(dim=-1) + lo
+        for b in range(B):
+            for g in range(G):
+                zT[b, g, :, 512 * 41:512 * 42] = zT[b, g, :, int(best[b, g])].unsqueeze(1)
+    P = hip_attend.merged_partitions(B * G, S, h)
+    assert plans.one_launch(B * G, lo, hi, L, k, h, P)
+    outs, ws = [], nat.Workspace()
+    for rows in (False, True):
+        got = sparse_decode_step_kernel(q, q_pre, K, V, zT.clone(), wq, wk, req.fixed_rows, req.off_lo, lo, hi, k, S,
+                                        k_pre_new=k_new, write_col=req.write_col, return_rows=rows, canonical_order=True,
+                                        partitions=P, workspace=ws)
+        torch.cuda.synchronize()
+        assert int(ws.bytes(gpu, 0, "state").abs().sum()) == 0, f"rows={rows}: the select state left dirty"
+        outs.append(got[0] if rows else got)
+    assert torch.equal(outs[0], outs[1])
+    u_out = torch.empty(B, G, 32, dtype=torch.float32, device=gpu)
+    s = hip_score.score_grouped(zT, lo, hi, q_cat=q_pre.reshape(B, G, h * 128).contiguous(), wq_t=wq, u_out=u_out)
+    torch.cuda.synchronize()
+    s = s.cpu().numpy()
+    for g in range(G):
+        recomputed, stored, crowd, _ = plans.list_paths(s[0, g], B * G, lo, hi, k)
+        assert (recomputed > 0) == (kind != "stored") and (stored > 0) == (kind != "recomputed") and crowd <= 8192, \
+            f"group {g}: {recomputed} tiles recomputed, {stored} stored, {crowd} keys in the threshold's bin"
+    want = exact.select_rows(s, lo, hi, L, k, order="position")
+    pos = (got[1].view(B, G, S) - req.offsets).cpu().numpy()
+    assert np.array_equal(pos, want)
+    i = torch.from_numpy(want).to(gpu).long().unsqueeze(-1).expand(-1, -1, -1, 128)
+    kk, vv = K.gather(2, i).double(), V.gather(2, i).double()
+    p = torch.softmax(torch.matmul(q[:, :, :, 0].double(), kk.transpose(2, 3).contiguous()) / math.sqrt(128), dim=-1)
+    check_out(outs[0], torch.matmul(p, vv).cpu().numpy(), f"{kind} L={L}")
+
+
 @pytest.mark.parametrize("B,G,h,L,rho,dtype", [
-    (1, 2, 2, 131072 + 68, 1 / 32, torch.bfloat16),   # every tile's keys stored
+    (1, 8, 2, 131072, 1 / 32, torch.bfloat16),        # eight sub-tiles per score workgroup
+    (1, 4, 2, 131072 + 68, 1 / 32, torch.bfloat16),   # the longest row
     (1, 2, 2, 40003, 1 / 32, torch.bfloat16),         # ragged: the last block partly past the row
     (2, 2, 4, 70000, 1 / 32, torch.float32),
     (1, 8, 2, 32768, 1 / 32, torch.bfloat16),
     (1, 3, 2, 30001, 1 / 8, torch.float32),
 ])
-@pytest.mark.parametrize("kind", ["common", "third", "equal"])
+@pytest.mark.parametrize("kind", ["common", "some", "equal"])
 def test_rows_that_crowd_one_first_digit(gpu, B, G, h, L, rho, dtype, kind):
     """More than 8192 keys share the threshold's first digit: index rows with a common part (two radix passes), such
-    rows in a random third of the 512-column blocks (their tiles' keys stored or listed, the others' lists complete) and
+    rows in nearly half of the 512-column blocks (their tiles' keys stored or listed, the others' lists complete) and
     equal rows (three passes, ties by index). The fused step equals the step that returns its rows, bit for bit (past
-    32768 candidates the tiled select, which reads stored scores), and those rows equal the oracle's."""
+    32768 candidates the tiled select, which reads stored scores), and those rows equal the oracle's; plans.list_paths
+    shows that the row crowds and which passes follow."""
     from attention_lab import _native as nat
     C = -(-L // 8) * 8
     ws = nat.Workspace()
     K, V, q, q_pre, k_pre_new, zT, idx = setup(gpu, B=B, G=G, h=h, C=C, seed=L + h)
     req = prepare_request(B, G, C, valid_length=L, query_position=L - 1, rho=rho, device=gpu)
     lo, hi = req.layout.candidate_lo, req.layout.candidate_hi
-    # a common part along u, so that every score moves by about four of its standard deviations
+    # a common part along u that moves every score by 1.125 times a power of two, at least 40 standard deviations: into
+    # the middle of a first-digit bin (a quarter octave, nine deviations there)
     u = torch.einsum("bgd,gdr->bgr", q_pre.float().reshape(B, G, -1).cpu(), idx.wq_t_scaled.float().cpu()).to(gpu)
-    part = (4.0 * u / u.norm(dim=-1, keepdim=True))[..., None]
+    n = u.norm(dim=-1, keepdim=True)
+    part = (1.125 * torch.exp2(torch.ceil(torch.log2(40.0 * n))) * u / (n * n))[..., None]
     z = zT.float()
     if kind == "common":
         z = z + part
-    elif kind == "third":
-        blocks = torch.rand(-(-C // 512), generator=torch.Generator().manual_seed(L)) < 1 / 3
+    elif kind == "some":
+        blocks = torch.rand(-(-C // 512), generator=torch.Generator().manual_seed(L)) < 0.45
         z = z + part * blocks.repeat_interleave(512)[:C].to(gpu)
     else:
         z[..., lo:hi] = z[..., lo:lo + 1]
     zT = z.to(dtype)
     wq, wk, qp, kn = (t.to(dtype) for t in (idx.wq_t_scaled, idx.wk, q_pre, k_pre_new))
+    P = hip_attend.merged_partitions(B * G, req.selected_count, h)
+    assert plans.one_launch(B * G, lo, hi, L, req.k, h, P)
     outs = []
     for rows in (False, True):
         got = sparse_decode_step_kernel(q, qp, K, V, zT.clone(), wq, wk, req.fixed_rows, req.off_lo, lo, hi, req.k,
                                         req.selected_count, k_pre_new=kn, write_col=req.write_col, return_rows=rows,
-                                        canonical_order=True, workspace=ws)
+                                        canonical_order=True, partitions=P, workspace=ws)
         torch.cuda.synchronize()
         assert int(ws.bytes(gpu, 0, "state").abs().sum()) == 0, f"rows={rows}: the select state left dirty"
         outs.append(got[0] if rows else got)
     assert torch.equal(outs[0], outs[1])
     pos = (got[1].view(B, G, req.selected_count) - req.offsets).cpu().numpy()
+    s = hip_score.score_grouped(zT, lo, hi, q_cat=qp.reshape(B, G, h * 128).contiguous(), wq_t=wq,
+                                u_out=torch.empty(B, G, 32, dtype=torch.float32, device=gpu))
+    torch.cuda.synchronize()
+    s = s.cpu().numpy()
+    assert np.array_equal(pos, exact.select_rows(s, lo, hi, L, req.k, order="position"))
+    for g in range(G):
+        _, stored, crowd, crowd2 = paths = plans.list_paths(s[0, g], B * G, lo, hi, req.k)
+        assert stored > 0 and crowd > 8192 and (crowd2 > 8192) == (kind == "equal"), paths
     if kind == "equal":
         want = np.concatenate([np.arange(lo + req.k), np.arange(hi, L)])
         assert (pos == want).all()
