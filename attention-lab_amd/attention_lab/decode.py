@@ -277,12 +277,7 @@ def sparse_decode_step_kernel(q_main, q_pre, k_cache, v_cache, zT, wq_t_scaled, 
             raise ValueError(f"write_col={write_col} must lie in [0, C) and outside [lo, hi)")
     else:
         wc = 0
-    if partitions is not None:
-        P = int(partitions)
-    elif k > 0:
-        P = hip_attend.merged_partitions(B * G, S, h, hip_attend.one_launch_step(h, hi - lo, return_rows))
-    else:
-        P = hip_attend.sparse_partitions(B * G, S, h)
+    P = hip_attend.step_partitions(B * G, S, h, hi - lo, k, bool(return_rows)) if partitions is None else int(partitions)
     sc = float(1.0 / math.sqrt(d) if scale is None else scale)
     order = nat.ORDER_POSITION if canonical_order else nat.ORDER_SCORE
     nbytes = nat.step_workspace_bytes(B, G, h, lo, hi, legal, k, P)

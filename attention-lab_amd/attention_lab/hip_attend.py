@@ -10,6 +10,7 @@ both on the same kernel.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -233,6 +234,15 @@ def one_launch_step(h: int, candidates: int, rows_returned: bool) -> bool:
     limit), at most 131072 candidates. A step that misses a further condition there (an unaligned table, k past about
     0.4 of the candidates, more than 128 score workgroups per row) takes this rule's P too."""
     return not rows_returned and h in (1, 2, 4) and candidates <= 131072
+
+
+@functools.lru_cache(maxsize=1024)
+def step_partitions(BG: int, rows: int, h: int, candidates: int, k: int, rows_returned: bool) -> int:
+    """The fused step's split-K count, a function of its sizes alone (every layer of a step asks for the same one): the
+    merged rule of the launches it runs, or, with nothing selected (k = 0, no select state), the combine kernel's."""
+    if k == 0:
+        return sparse_partitions(BG, rows, h)
+    return merged_partitions(BG, rows, h, one_launch_step(h, candidates, rows_returned))
 
 
 def dense_partitions(BG: int, length: int) -> int:

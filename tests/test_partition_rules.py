@@ -6,7 +6,7 @@ from __future__ import annotations
 
 import pytest
 
-from attention_lab.hip_attend import merged_partitions, one_launch_step, sparse_partitions
+from attention_lab.hip_attend import merged_partitions, one_launch_step, sparse_partitions, step_partitions
 
 
 @pytest.mark.parametrize("BG,S,h,want", [
@@ -55,3 +55,5 @@ def test_which_steps_run_in_one_launch():
     assert one_launch_step(4, 32700, False) and one_launch_step(1, 131072, False)
     assert not one_launch_step(4, 32700, True) and not one_launch_step(4, 131073, False)
     assert not any(one_launch_step(h, 32700, False) for h in (3, 5, 6, 7, 8))
+    assert step_partitions(96, 1092, 4, 32700, 1024, False) == 1 and step_partitions(96, 1092, 4, 32700, 1024, True) == 2
+    assert step_partitions(96, 1092, 4, 0, 0, False) == sparse_partitions(96, 1092, 4)
