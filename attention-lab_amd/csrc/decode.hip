@@ -125,9 +125,8 @@ int sparse_decode_step_impl(const uint16_t* q_main, const uint16_t* K, const uin
         }
     }
     // Stored scores are read only by the tiled select and by score order (which reads the picks' scores back to sort
-    // them); the list select in position order recomputes the rare tile it needs from the table and u, so the score
-    // kernel then writes key lists only. The
-    // keys of a tile whose list was cut go where the scores would (write_key_list).
+    // them). In position order the score kernel writes key lists only, and the keys of a tile whose list was cut where the
+    // scores would go (write_key_list); the list select recomputes the rare other tile it needs from the table and u.
     const bool store_scores = plan.cap == 0 || order == ATTNLAB_ORDER_SCORE;
     if (!store_scores) {
         lists.keys = reinterpret_cast<uint32_t*>(scores);

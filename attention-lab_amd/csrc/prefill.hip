@@ -399,8 +399,9 @@ __global__ __launch_bounds__(256) void project_keys_mfma(ProjectArgs a) {
 //   O^T += V^T P^T A = 32 dims x 16 keys read from the row-major V tile by the transposing LDS read, B = P^T
 // O^T keeps each row's 128 outputs in the lanes of that row, so rescaling needs no exchange. K and V tiles are copied
 // into LDS without passing through registers, one block ahead (two pairs of tiles, one barrier per block).
-// What bounds it: power. At B=1, G=8, h=4, T=L=8192 it runs 524 us (1.04 PFLOP/s) at a clock of 2.04 GHz (2.4 GHz at
-// light load); forms that need fewer cycles (all operand reads issued ahead, the next block's S^T under this block's
+// What bounds it: power. At B=1, G=8, h=4, T=L=8192 it runs 524-529 us (1.04 PFLOP/s) at a clock of 2.04 GHz (2.4 GHz at
+// light load; 1.87 under counters, where the matrix cores are busy 49 % of the cycles and no LDS access conflicts); forms
+// that need fewer cycles (all operand reads issued ahead, the next block's S^T under this block's
 // softmax) or more (one workgroup of 8 waves, 2.27 GHz) end at the same time within 2 %, and one workgroup per CU at
 // 2.41 GHz takes 657 us. The form before this one (K and V through registers, V transposed by 4-byte LDS stores, two
 // barriers per block) took 642 us; the 1000-token chunk after 29011 (h=2) went from 309 to 264 us.

@@ -402,8 +402,8 @@ __global__ __launch_bounds__(256) void score_scan_fused(ScoreArgs a) {
         a.sink[(size_t)lin * 256 + tid] = fx;
         return;
     }
-    // a.out null (key lists only, the fused step's position order): no score is stored; the list select recomputes
-    // the few tiles it needs from the table
+    // a.out null (key lists only, the fused step's position order): no score is stored; the list select reads a
+    // cut list's tile from its stored keys (write_key_list) and recomputes the few others it needs from the table
     float* o = a.out ? a.out + (size_t)bg * a.out_stride - lo : nullptr;
     uint32_t lkey[2 * NSUB];   // this thread's keys (columns cb0 + s * sstride + 2 tid + e), kept for the list
     uint32_t lvalid = 0u;

@@ -328,8 +328,8 @@ __device__ __forceinline__ void radix_stored(const ListRow& r, const ListLds& L,
 // equal to it. Called by every thread with the same b1 and krem. A wave takes 512 table columns at a time, which lie in one
 // tile. SCORES: from the stored scores. Else, where the tile's list was cut, from its stored keys, several blocks in flight;
 // where it is complete down to b1, from the list; else recomputed. Reading 4 stored bytes a candidate against recomputing
-// it from 64 in every workgroup of the row, per layer: index rows with a common part, B=8 h=4 at 32K 190.8 -> 63.7 us, B=2
-// h=2 at 128K 556 -> 119; equal rows 153 -> 69 and 428 -> 125. Rows that crowd no digit pay nothing at 32K (B=1 18.9 both)
+// it from 64 in every workgroup of the row, per layer: rows whose keys all lie in one bin, B=8 h=4 at 32K 146 -> 62 us, B=2
+// h=2 at 128K 405 -> 100; equal rows 153 -> 69 and 428 -> 125. Rows that crowd no digit pay nothing at 32K (B=1 18.9 both)
 // and up to 0.5 us past 32768 candidates (B=1 64K 26.0 -> 26.5).
 template <int THREADS, int WORDS, bool SCORES>
 __device__ __forceinline__ void radix_bitmap(const ListRow& r, const ListLds& L, uint32_t b1, uint32_t krem) {
