@@ -7,7 +7,7 @@
 // is a 1 KiB contiguous run of HBM. The loads are issued before u is built, so the prologue (16-32 KiB of weights,
 // L2-resident after the first block) hides under the HBM latency instead of adding to it.
 //
-// Lightning mode (the north_star generalisation; no reference kernel): keys are stored one r-vector per position
+// Lightning mode (a generalisation; no reference kernel): keys are stored one r-vector per position
 // [B,KG,Lk,r] (64 bytes of fp16/bf16 per position), four lanes share a position with 16 bytes each, the per-head
 // partial dot products of a quad's four keys are reduced and transposed with two DPP steps, and ReLU and the head
 // weights are applied in fp32.

@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the sparse-decode hot path on one MI355X.
 
-Workload (its attention geometry): a Qwen3-8B-shaped stack of 36 layers, each with its own
+Workload (a Qwen3-8B serving shape's attention geometry): a Qwen3-8B-shaped stack of 36 layers, each with its own
 bf16 K/V cache [16, 8, 32768, 128] and bf16 index table [16, 8, 32, 32768] resident in HBM (~87 GB), 4 query heads
 per KV group, one r=32 grouped indexer per layer (seeded as the reference seeds them), rho = 1/32 -> k = 1024 of the
 32700 candidates, S = 1092 rows per (b, g). Synthetic data: K, V, index keys, queries ~ N(0, 1).
@@ -70,23 +70,23 @@ def parse_args():
                     help="per-kernel means of every counter in the rocprofv3 --pmc output directories given (FETCH_SIZE "
                          "and WRITE_SIZE also in bytes, scaled by the 256 MiB calibration copy); no GPU needed")
     ap.add_argument("--sweeps", nargs="?", const="all", choices=("all", "score", "attend"),
-                    help="instead of the bench line: the microbenchmark sweeps of BASELINE configs[1] (lightning score "
-                         "+ top-k) and configs[2] (gather-free attend vs dense), one JSON line per case")
+                    help="instead of the bench line: the microbenchmark sweeps of the lightning score "
+                         "+ top-k and of the gather-free attend vs dense, one JSON line per case")
     ap.add_argument("--c4", action="store_true",
-                    help="instead of the bench line: BASELINE configs[3], a random-init Qwen3-1.7B-shaped model read "
+                    help="instead of the bench line: a random-init Qwen3-1.7B-shaped model read "
                          "through the wrapper: 8192-token prompt, 128 greedy steps on the full read, the same tokens on "
                          "the sparse read (rho = 1/32); per-step logits compared, one JSON line")
     ap.add_argument("--c4-steps", type=int, default=128)
     ap.add_argument("--c4-prompt", type=int, default=8192)
     ap.add_argument("--c5", action="store_true",
-                    help="instead of the bench line: BASELINE configs[4], a random-init Qwen3-8B-shaped model read "
+                    help="instead of the bench line: a random-init Qwen3-8B-shaped model read "
                          "through the wrapper at batch 16 x 32K context (uniform random ids): 64 greedy steps on the "
                          "full read, the same tokens on the sparse read (rho = 1/32), eager per-step times; one JSON "
                          "line")
     ap.add_argument("--c5-steps", type=int, default=64)
     ap.add_argument("--c5-context", type=int, default=32768)
     ap.add_argument("--c5-batch", type=int, default=16)
-    ap.add_argument("--c5-chunk", type=int, default=2048, help="prefill chunk of the configs[4] run")
+    ap.add_argument("--c5-chunk", type=int, default=2048, help="prefill chunk of the Qwen3-8B-shaped run")
     ap.add_argument("--p0", action="store_true",
                     help="instead of the bench line: the reference's P0 score bench (bench/p0_score_kernel.py) on the "
                          "HIP score ops: batch 1, G=8, h=2, 28 rotating layers per length; PyTorch chain / score-only "
@@ -663,7 +663,7 @@ def run_prefill_score(torch, dev, reps=10):
 
 
 # ---------------------------------------------------------------------------------------------------------------------
-# microbenchmark sweeps of configs[1] and configs[2]
+# microbenchmark sweeps: lightning score + top-k, gather-free attend vs dense
 # ---------------------------------------------------------------------------------------------------------------------
 COLD_BYTES = 1 << 30   # rotate over input copies of at least this many bytes, so reads come from HBM, not the caches
 
@@ -694,7 +694,7 @@ def time_rotating(torch, launch, copies, reps=10):
 
 
 def sweep_lightning_topk(torch, dev, emit):
-    """batch {1, 8, 32} x L {4K, 16K, 64K, 128K}, 4 index heads of r = 32, fp16 keys ~ N(0, 1/32),
+    """Lightning score + top-k: batch {1, 8, 32} x L {4K, 16K, 64K, 128K}, 4 index heads of r = 32, fp16 keys ~ N(0, 1/32),
     q ~ N(0, 1), w ~ U(0, 1), ReLU, k = L / 32; 2 % of each row's positions get +3 sigma of that row's scores before
     the top-k. Key groups G_I = 1 (one shared index per sequence) and 8 (one per KV group)."""
     from attention_lab import _native as nat
@@ -769,7 +769,7 @@ def sweep_lightning_topk(torch, dev, emit):
 
 
 def sweep_attend(torch, dev, emit):
-    """L = 32K, 8 KV groups x 2 query heads, d = 128, bf16 K/V ~ N(0, 1); rows = 4 sinks + the 128 most
+    """Gather-free attend vs dense: L = 32K, 8 KV groups x 2 query heads, d = 128, bf16 K/V ~ N(0, 1); rows = 4 sinks + the 128 most
     recent positions + k uniform picks from the rest (S = 132 + k), k in {64, 256, 1024, 2048}, batch {1, 16}, rows
     sorted and unsorted; against the dense decode kernel at the same shape."""
     from attention_lab import _native as nat
@@ -821,7 +821,7 @@ def sweep_attend(torch, dev, emit):
 
 
 def qwen3_1p7b(torch, dev, seed):
-    """BASELINE configs[3]'s model shape with random bf16 weights ~ N(0, 0.02) (transformers' own init), on `dev`."""
+    """The Qwen3-1.7B shape with random bf16 weights ~ N(0, 0.02) (transformers' own init), on `dev`."""
     from transformers import Qwen3Config, Qwen3ForCausalLM
     cfg = Qwen3Config(vocab_size=151936, hidden_size=2048, intermediate_size=6144, num_hidden_layers=28,
                       num_attention_heads=16, num_key_value_heads=8, head_dim=128, max_position_embeddings=40960,
@@ -837,7 +837,7 @@ def qwen3_1p7b(torch, dev, seed):
 
 
 def qwen3_8b(torch, dev, seed):
-    """BASELINE configs[4]'s model shape (36 layers, hidden 4096, 32q/8kv, d=128, FFN 12288, vocab 151936) with random
+    """The Qwen3-8B shape (36 layers, hidden 4096, 32q/8kv, d=128, FFN 12288, vocab 151936) with random
     bf16 weights ~ N(0, 0.02) (transformers' own init), on `dev`."""
     from transformers import Qwen3Config, Qwen3ForCausalLM
     cfg = Qwen3Config(vocab_size=151936, hidden_size=4096, intermediate_size=12288, num_hidden_layers=36,
@@ -864,7 +864,7 @@ def logit_agreement(torch, a, b):
 
 
 def run_c5(torch, dev, args):
-    """configs[4] through the wrapper on the HIP kernels: one chunked prefill of B x L uniform random ids (index table
+    """The Qwen3-8B shape through the wrapper on the HIP kernels: one chunked prefill of B x L uniform random ids (index table
     built on the way), greedy decode on the full read (A), rollback, the same tokens (teacher-forced) on the sparse
     read (D0, rho = 1/32), and a few steps with k0 = capacity (every candidate selected, which must equal A). Per-step
     times are eager wall clock (the model's own layers launch from Python), each step ending in a synchronize."""
@@ -968,7 +968,7 @@ def run_c5(torch, dev, args):
     res["tok_s_sparse"] = round(B * 1e3 / res["decode_ms_sparse"], 1)
     res["sparse_speedup"] = round(res["decode_ms_full"] / res["decode_ms_sparse"], 3)
     print(json.dumps({
-        "workload": f"configs[4]: random-init Qwen3-8B shape (36 layers, hidden 4096, 32q/8kv, d=128, FFN 12288, "
+        "workload": f"random-init Qwen3-8B shape (36 layers, hidden 4096, 32q/8kv, d=128, FFN 12288, "
                     f"vocab 151936, bf16 ~ N(0, 0.02)), batch {B} x {L}-token uniform random context, {steps} greedy "
                     f"steps on the full read, the same tokens on the sparse read (rho={args.rho}, one r=32 grouped "
                     f"indexer per layer) and {n_all} on the sparse read with k0 = capacity; whole model on the GPU, "
@@ -1200,7 +1200,7 @@ def run_p1(torch, dev, args):
 
 
 def run_c4(torch, dev, args):
-    """configs[3] through the wrapper on the HIP kernels: greedy decode on the full read (A); the same tokens on the
+    """The Qwen3-1.7B shape through the wrapper on the HIP kernels: greedy decode on the full read (A); the same tokens on the
     sparse read (D0, rho = 1/32) and on the sparse read with k0 = capacity (every candidate selected, which must
     equal A); the full read against the unwrapped model in float32 with transformers' eager attention."""
     from attention_lab.qwen_wrap import LabRunner, make_state, unwrap_model, wrap_model
@@ -1274,7 +1274,7 @@ def run_c4(torch, dev, args):
         ref = ref_model(input_ids=ids, use_cache=False, logits_to_keep=steps + 1).logits[0, 1:].float()
         res["full_vs_float32_eager_reference"] = compare(full_logits, ref)
     print(json.dumps({
-        "workload": f"configs[3]: random-init Qwen3-1.7B shape (28 layers, hidden 2048, 16q/8kv, d=128, FFN 6144, "
+        "workload": f"random-init Qwen3-1.7B shape (28 layers, hidden 2048, 16q/8kv, d=128, FFN 6144, "
                     f"vocab 151936, bf16 ~ N(0, 0.02)), {T0}-token uniform prompt, {steps} greedy steps on the full "
                     f"read; the same tokens (teacher-forced) on the sparse read (rho={args.rho}, k0={k0}, one r=32 "
                     f"grouped indexer per layer) and on the sparse read with k0 = capacity; whole model on the GPU, "
@@ -1348,7 +1348,7 @@ def _cpu_time(fn, budget_s, min_n=2):
 
 
 def _c1_inputs(torch, seed=0, B=1, G=8, h=2, L=2048, r=32, d=128):
-    """configs[0] on the CPU: one Qwen3-0.6B-shaped layer, L=2048, 16q/8kv, bf16 K/V ~ N(0,1), grouped r=32 indexer."""
+    """On the CPU: one Qwen3-0.6B-shaped layer, L=2048, 16q/8kv, bf16 K/V ~ N(0,1), grouped r=32 indexer."""
     from attention_lab.indexer import GroupedIndexer
     g = torch.Generator().manual_seed(seed)
     t = lambda *sh: torch.randn(*sh, generator=g).to(torch.bfloat16)  # noqa: E731
@@ -1358,7 +1358,7 @@ def _c1_inputs(torch, seed=0, B=1, G=8, h=2, L=2048, r=32, d=128):
 
 
 def _lightning_cpu(torch, keys, q, w, k):
-    """configs[1]'s indexer score + top-k on the CPU: s = sum_i w_i ReLU(q_i . key_t), then torch.topk (float32)."""
+    """The lightning indexer's score + top-k on the CPU: s = sum_i w_i ReLU(q_i . key_t), then torch.topk (float32)."""
     s = torch.einsum("gir,gtr->git", q, keys).clamp_min_(0.0)
     s = torch.einsum("gi,git->gt", w, s)
     return torch.topk(s, k, dim=-1)
@@ -1366,8 +1366,8 @@ def _lightning_cpu(torch, keys, q, w, k):
 
 def cpu_baseline(torch, ls, budget_s, layers_in_step):
     """The reference's op sequence (oracle/ref_path.py: bf16 matmul score, torch.topk, cat, index_select, SDPA) on the
-    host cores: layer 0 of the bench shape at all usable CPUs (the headline `value`) and at 1 thread, plus BASELINE's
-    B=1 legs: configs[0] (sparse and dense step at L=2048) and configs[1] (lightning score + top-k, L = 4K..32K)."""
+    host cores: layer 0 of the bench shape at all usable CPUs (the headline `value`) and at 1 thread, plus
+    B=1 legs: a sparse and a dense step at L=2048, and the lightning score + top-k at L = 4K..32K."""
     from oracle import ref_path
     info = cpu_info()
     threads_all = info["usable_cpus"]
@@ -1417,7 +1417,7 @@ def cpu_baseline(torch, ls, budget_s, layers_in_step):
                 "sample": (f"{res['all']['layer_steps']} layer-steps of layer 0 (B={ls.B}, L={ls.L}, G={ls.G}, "
                            f"h={ls.h}, k={ls.k}) through the reference's op sequence in bf16 (matmul, torch.topk, "
                            f"cat, index_select, SDPA) on {threads_all} threads, scaled to {layers_in_step} layers; "
-                           f"the same at 1 thread in one_thread; B=1 legs of configs[0] and configs[1] in both")})
+                           f"the same at 1 thread in one_thread; B=1 legs (step at 2K, lightning score + top-k) in both")})
     return res, out_cpu, rows_cpu
 
 

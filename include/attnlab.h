@@ -125,7 +125,7 @@ int attnlab_project_keys_f32(const float* k_pre, int64_t k_bg_stride, int64_t k_
                              float* zT, int B, int G, int T, int r, int d, int C, int col0, void* stream);
 
 /*
- * Lightning-indexer score (no reference kernel: the generalisation north_star names; the grouped score of
+ * Lightning-indexer score (no reference kernel: a generalisation; the grouped score of
  * indexer.py:27-29 is the special case nh=1, w=1, relu=0, keys transposed):
  *   out[b,kg,t] = sum_i w[b,kg,i] * act(sum_j q[b,kg,i,j] * key[b,kg,t,j])   for t in [lo, hi), act = ReLU or identity
  * keys: [B,KG,Lk,r] (row layout, one r-vector per position) in key_dtype (ATTNLAB_DT_F16 or ATTNLAB_DT_BF16);
@@ -137,8 +137,8 @@ int attnlab_score_lightning(const uint16_t* keys, int key_dtype, const float* q,
                             void* stream);
 
 /*
- * Batched (prefill) lightning-indexer score on the matrix cores: the T-query form of attnlab_score_lightning, the
- * "batched/prefill score contraction" north_star puts on MFMA (no reference kernel; per query it is the formula of
+ * Batched (prefill) lightning-indexer score on the matrix cores: the T-query form of attnlab_score_lightning
+ * (no reference kernel; per query it is the formula of
  * attnlab_score_lightning, and with nh=1, w=1, relu=0 the grouped score of indexer.py:27-29 for T queries):
  *   out[b,kg,t,m-lo] = sum_i w[b,kg,t,i] * act(sum_j q[b,kg,t,i,j] * key[b,kg,m,j])
  * for m in [lo, hi) and, when q_pos0 >= 0, m <= q_pos0 + t (causal: query t sits at position q_pos0 + t); entries

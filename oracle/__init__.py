@@ -10,8 +10,8 @@ Modules (each function cites the reference file:line it restates; paths relative
             metal_score.py:31-40, 84-89), top-k with lowest-index ties (decode.py:86-93 made deterministic), row list
             (decode.py:50-56, 86-93, 160-161), subset attention (metal_attend.py:262-273, reference.py:80-97), dense
             attention (reference.py:51-62, full.py:17-34), causal attention of a prefill chunk (reference.py:28-62,
-            legality mask), lightning score and its T-query prefill form with a causal bound (north_star formula,
-            no reference code)
+            legality mask), lightning score and its T-query prefill form with a causal bound (no reference
+            code)
   ref_path  the reference's torch op sequence on the CPU (matmul -> topk -> cat -> index_select -> SDPA), the timed
             CPU baseline
   weights   GroupedIndexer's seeded weights (indexer.py:38-45)

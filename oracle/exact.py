@@ -42,7 +42,7 @@ def project_keys(k_pre: np.ndarray, wk: np.ndarray) -> np.ndarray:
 def lightning_scores(keys: np.ndarray, q: np.ndarray, w: np.ndarray, lo: int, hi: int, relu: bool = True):
     """s[b,kg,t] = sum_i w[b,kg,i] * act(q[b,kg,i] . keys[b,kg,t]) for t in [lo, hi).
 
-    The north_star lightning indexer; with nh = 1, w = 1 and act = identity it is grouped_scores with the key table
+    The lightning indexer; with nh = 1, w = 1 and act = identity it is grouped_scores with the key table
     transposed (the reduction the tests use to pin it).
     """
     dots = np.einsum("bkir,bktr->bkit", q, keys[:, :, lo:hi])
@@ -56,7 +56,7 @@ def lightning_scores_batched(keys: np.ndarray, q: np.ndarray, w: np.ndarray, lo:
     """T queries per (b, kg): s[b,kg,t,m-lo] = lightning_scores of query t (q [B,KG,T,nh,r], w [B,KG,T,nh]) for m in
     [lo, hi); with q_pos0, query t sits at position q_pos0 + t and the entries m > q_pos0 + t are NaN (not scored).
 
-    The prefill form of the north_star lightning indexer (no reference code); one query is lightning_scores.
+    The prefill form of the lightning indexer (no reference code); one query is lightning_scores.
     """
     dots = np.einsum("bktir,bkmr->bktim", q, keys[:, :, lo:hi])
     if relu:

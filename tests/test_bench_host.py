@@ -126,7 +126,7 @@ def test_p0_p1_geometry_matches_the_reference_benches():
 
 def test_cpu_info_and_the_lightning_cpu_leg():
     """The CPU baseline's host facts (the CPUs the all-cores leg uses never exceed what the process may run on) and
-    its configs[1] leg, which must compute the lightning score + top-k the oracle defines."""
+    its lightning leg, which must compute the lightning score + top-k the oracle defines."""
     import numpy as np
     import torch
 
@@ -143,7 +143,7 @@ def test_cpu_info_and_the_lightning_cpu_leg():
 
 
 def test_topk_picks_the_tiled_kernels_by_row_length_and_count():
-    """hip_select.topk's automatic choice (also the configs[1] sweep's): tiled kernels for 32K..256K keys, except rows
+    """hip_select.topk's automatic choice (also the lightning sweep's): tiled kernels for 32K..256K keys, except rows
     of at most 32K keys when 128 or more of them fill half the chip as one workgroup each."""
     from attention_lab import hip_select
     assert not hip_select.use_tiled(1, 16384)

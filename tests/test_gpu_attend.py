@@ -2,7 +2,7 @@
 
 Preset tolerances (test_metal_attend.py:28-29): fp32 output vs the float64 masked-dense reference on the same bf16
 inputs, max |d| <= 5e-5 and relative norm <= 1e-5, for every partition count; the bf16 output within one bf16 ulp of
-the RNE of the fp32 output, >= 99% bitwise. north_star's looser bf16 bound (max 2e-2, mean 2e-3) is implied.
+the RNE of the fp32 output, >= 99% bitwise. The looser bf16 attention bound (max 2e-2, mean 2e-3) is implied.
 """
 from __future__ import annotations
 

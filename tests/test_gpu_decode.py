@@ -1,7 +1,7 @@
 """The whole sparse decode step (z column -> score -> top-k -> row list -> gather-free attend) against the oracle.
 
 Bars: row lists bit-exact against the oracle's top-k on the kernel's own fp32 scores; scores within 1e-5 of the
-float64 oracle; z column >= 99% bitwise equal to the RNE of the exact value; attention output within north_star's bf16
+float64 oracle; z column >= 99% bitwise equal to the RNE of the exact value; attention output within the bf16
 tolerance (max |d| <= 2e-2, mean |d| <= 2e-3) of the float64 subset attention over the same rows. Invariants from the
 reference's contracts: NaN poison in unselected or unwritten rows is inert, every candidate selected (k = M) equals
 the dense read, legal <= 68 degenerates to the dense read, rows are original positions.

@@ -1,8 +1,8 @@
 """Float32 index tables on the GPU: the trained bank's dtype (trained.py:11-18, 78-81) through the fp32 score, z
 column, query projection, bulk build and the fused decode step, against the float64 oracle.
 
-Bars, written here: scores and u within 1e-5 of the oracle on the same fp32 inputs (the north_star asks 1e-3
-relative); the z column and the bulk build, sums of d fp32 products stored unrounded, within 128 * 2^-24 of the exact value
+Bars, written here: scores and u within 1e-5 of the oracle on the same fp32 inputs (1e-3 relative is
+asked); the z column and the bulk build, sums of d fp32 products stored unrounded, within 128 * 2^-24 of the exact value
 relative to the sum of |terms| (the error bound of any summation order of d = 128 fp32 terms; a dropped or doubled
 term breaks it); row lists bit-exact against the oracle's top-k on the kernel's own fp32 scores;
 attention output within the bf16 bar (max |d| <= 2e-2, mean |d| <= 2e-3).

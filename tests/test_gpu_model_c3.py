@@ -1,4 +1,4 @@
-"""BASELINE configs[3] on the GPU through the wrapper: a random-init Qwen3-1.7B-shaped model (28 layers, hidden 2048,
+"""A whole model on the GPU through the wrapper: a random-init Qwen3-1.7B-shaped model (28 layers, hidden 2048,
 16q/8kv, head_dim 128, FFN 6144, vocab 151936, rope theta 1e6, bf16 weights ~ N(0, 0.02)), an 8192-token uniform
 prompt, then greedy decode steps (reference tests/test_qwen_wrapper.py:150-173 and :455-480, bench/model_numerics.py:
 54-146).
@@ -104,7 +104,7 @@ def test_configs3_qwen3_1p7b_8192_prompt(gpu):
 
 
 def test_configs3_partial_read_at_rho_1_32_touches_only_its_rows(gpu):
-    """configs[3] at its real budget: after the 8192-token prompt, one decode step at rho = 1/32 (k0 = 256 of 8125
+    """The same model at its real budget: after the 8192-token prompt, one decode step at rho = 1/32 (k0 = 256 of 8125
     candidates) in both row orders, with every layer's row list recorded. Each list holds S = 68 + k unique positions
     inside the legal range, F among them ([0, 4) and the last 64), the candidates inside [lo, hi); position order is
     strictly ascending, score order puts F first. Then every K/V row the step did not select is poisoned with NaN in

@@ -1,7 +1,7 @@
 """Causal prefill read on the matrix cores (attnlab_prefill_attend) against the float64 oracle and an fp32 reference.
 
 The reference's legality rule (reference.py:41-48): key j is legal for query t iff j <= its position and
-j < valid_length. Tolerances, written here: the north_star's bf16 attention bar, max |d| <= 2e-2 and mean |d| <= 2e-3
+j < valid_length. Tolerances, written here: the bf16 attention bar, max |d| <= 2e-2 and mean |d| <= 2e-3
 against the float64 oracle on the same bf16 inputs.
 """
 from __future__ import annotations

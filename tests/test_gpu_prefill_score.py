@@ -1,7 +1,7 @@
 """Batched (prefill) lightning score on the matrix cores against the oracle and against the one-query kernel.
 
 Tolerances, written here: fp32 scores against the float64 oracle on the same fp16/bf16 keys and fp32 queries, max |d|
-<= 1e-5 * max(1, max |ref|) and relative norm <= 1e-5 (north_star asks 1e-3 relative); against the one-query kernel
+<= 1e-5 * max(1, max |ref|) and relative norm <= 1e-5 (1e-3 relative is asked); against the one-query kernel
 (fp32 FMAs in another order) 2e-6 * max(1, max |score|). Entries past a query's causal bound must keep what `out`
 held (the kernel does not write them).
 """

@@ -1,7 +1,7 @@
 """Score kernels on the GPU against the oracle (contracts of the reference's tests/test_metal_score.py).
 
 Preset tolerances (test_metal_score.py:27): fp32 scores vs the float64 oracle on the same bf16 inputs, max |d| <= 1e-5
-and relative norm <= 1e-5 (north_star asks only 1e-3 relative); z column within one bf16 ulp (2^-8 relative) of the
+and relative norm <= 1e-5 (only 1e-3 relative is asked); z column within one bf16 ulp (2^-8 relative) of the
 PyTorch bf16 path and >= 90% bitwise equal to it; the RNE of the exact z bitwise in >= 99%.
 """
 from __future__ import annotations
