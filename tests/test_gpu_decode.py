@@ -415,7 +415,7 @@ def _shape_scores(zT, lo, hi, case):
 @pytest.mark.parametrize("B,h,C,L,rho", [
     (2, 2, 8192 + 64, 8192, 1 / 8),       # one 512-column sub-tile per score workgroup, M < 8192
     (1, 2, 16384 + 64, 16384, 1 / 16),    # M > 8192: an all-equal row overflows the LDS candidates
-    (16, 4, 16384, 16384, 1 / 32),        # two sub-tiles per score workgroup
+    (16, 4, 16384, 16384, 1 / 32),        # eight sub-tiles per score workgroup
 ])
 def test_list_select_on_hard_distributions(gpu, case, B, h, C, L, rho):
     K, V, q, q_pre, k_pre_new, zT, idx = setup(gpu, B=B, h=h, C=C, seed=L + B)
@@ -633,7 +633,7 @@ def test_in_kernel_partition_merge_equals_the_combine_kernel(gpu, G, h, P):
 @pytest.mark.parametrize("B,G,h,C,L,rho,case,P", [
     (1, 8, 2, 2048 + 64, 2048, 1 / 32, None, None),          # config 1
     (1, 8, 2, 32768 + 64, 32768, 1 / 32, None, None),        # B=1 at 32K: partitions split each row
-    (16, 8, 4, 16384, 16384, 1 / 32, None, None),            # two sub-tiles per score workgroup
+    (16, 8, 4, 16384, 16384, 1 / 32, None, None),            # eight sub-tiles per score workgroup
     (2, 8, 4, 8192 + 64, 8192, 1 / 8, "skewed_tile", None),  # an incomplete list: its tile recomputed
     (1, 8, 2, 16384 + 64, 16384, 1 / 16, "all_equal", None), # bin b1 past the LDS candidates: radix passes
     (2, 8, 2, 8192 + 64, 8192, 1 / 8, "seven_values", None), # ties at the threshold

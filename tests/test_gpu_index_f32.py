@@ -194,7 +194,7 @@ def _shape_table(zT, lo, hi, case):
 @pytest.mark.parametrize("B,h,C,L,rho", [
     (2, 2, 8192 + 64, 8192, 1 / 8),       # one 512-column sub-tile per score workgroup, M < 8192
     (1, 2, 16384 + 64, 16384, 1 / 16),    # M > 8192: an all-equal row overflows the select's LDS candidates
-    (16, 4, 16384, 16384, 1 / 32),        # two sub-tiles per score workgroup
+    (16, 4, 16384, 16384, 1 / 32),        # eight sub-tiles per score workgroup
 ])
 def test_step_list_select_on_hard_distributions(gpu, case, B, h, C, L, rho):
     """The float32 one-launch score's key lists through the list select, in both row orders, bit-exact against the
